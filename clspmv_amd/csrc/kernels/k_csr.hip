@@ -5,11 +5,9 @@
 //  * csr_vector<L>: L lanes per row (L = 2..64 picked from the mean row
 //    length), DPP/shuffle group reduction.  The reference's CSR-vector uses
 //    a fixed 32-lane "warp" per row (A/kernels/spmv_csr_vector.cl:4-40).
-//  * csr_adaptive: row blocks planned on the host so that every wave gets a
-//    balanced amount of work whatever the row-length distribution:
-//      STREAM  rows [r0,r1) with <= 512 nnz in total and no row longer than
-//              64: the wave streams the block's nnz range into LDS with
-//              fully coalesced loads (8 per lane), then lane j sums row j;
+//  * csr_adaptive: rows of at most 64 entries in row groups (csr_group
+//    below: one to sixteen lanes per row, the entries of 64 lanes
+//    interleaved at upload), longer rows by host-planned blocks:
 //      VECTOR  one row of 65..1024 nnz: the wave strides the row and
 //              reduces across its 64 lanes;
 //      LONG    one 1024-nnz chunk of a longer row: the wave's partial is
@@ -17,6 +15,8 @@
 //              long row in order (deterministic, no atomics).
 #include "kcommon.hpp"
 #include "launch.hpp"
+
+#include <type_traits>
 
 namespace clspmv {
 namespace dev {
@@ -60,60 +60,159 @@ __global__ __launch_bounds__(256) void csr_vector_kernel(const int* __restrict__
     if (lane == 0 && e > s) y[row] += acc;
 }
 
-__global__ __launch_bounds__(256) void csr_adaptive_kernel(const int* __restrict__ rp, const int* __restrict__ col,
-                                                           const float* __restrict__ val,
-                                                           const int4* __restrict__ blocks, int nblocks,
-                                                           const float* __restrict__ x, float* __restrict__ y,
-                                                           double* __restrict__ carry) {
-    __shared__ float lds[4][kCsrStreamMaxNnz];
-    const int wid = threadIdx.x >> 6;
+// One block of a long row (VECTOR or LONG, DevCsrAdaptive::blocks), by one
+// wave.
+__device__ __forceinline__ void csr_long_block(const DevCsrAdaptive& m, int b, const float* __restrict__ x,
+                                               float* __restrict__ y, int lane) {
+    const int4 blk = m.blocks[b];
+    const int row = blk.x, tag = blk.y, n0 = blk.z, n1 = blk.w;
+    const int* __restrict__ col = m.col;
+    const float* __restrict__ val = m.val;
+    float acc = 0.f;
+    int k = n0 + lane;
+    for (; k + 192 < n1; k += 256) {
+        int c0 = ld_stream(col + k), c1 = ld_stream(col + k + 64), c2 = ld_stream(col + k + 128),
+            c3 = ld_stream(col + k + 192);
+        float v0 = ld_stream(val + k), v1 = ld_stream(val + k + 64), v2 = ld_stream(val + k + 128),
+              v3 = ld_stream(val + k + 192);
+        acc = fmaf(v0, x[c0], acc);
+        acc = fmaf(v1, x[c1], acc);
+        acc = fmaf(v2, x[c2], acc);
+        acc = fmaf(v3, x[c3], acc);
+    }
+    for (; k < n1; k += 64) acc = fmaf(ld_stream(val + k), x[ld_stream(col + k)], acc);
+    acc = wave_sum(acc);
+    if (lane == 0) {
+        if (tag < 0)
+            m.carry[-tag - 1] = (double)acc;
+        else
+            y[row] += acc;
+    }
+}
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x2 __attribute__((ext_vector_type(2)));
+
+// kCsrPairs pairs of a wave from pair p on (those past the wave's last are
+// skipped, wave-uniform): two values and two columns per lane and pair.
+template <int MODE>
+struct CsrPairs {
+    typedef typename std::conditional<MODE == kCsrWide, i32x2, unsigned>::type C;
+    f32x2 v[kCsrPairs];
+    C c[kCsrPairs];
+    __device__ __forceinline__ void load(const f32x2* __restrict__ val, const char* __restrict__ col, int p, int pairs,
+                                         int lane) {
+        const C* cp = reinterpret_cast<const C*>(col);
+#pragma unroll
+        for (int u = 0; u < kCsrPairs; ++u)
+            if (p + u < pairs) {
+                v[u] = __builtin_nontemporal_load(val + (size_t)(p + u) * 64 + lane);
+                c[u] = __builtin_nontemporal_load(cp + (size_t)(p + u) * 64 + lane);
+            }
+    }
+};
+
+// A wave's pairs times x (the first kCsrPairs of them loaded by the caller):
+// the lane's row holds entries 2 L p + 2 t and + 1 of pair p; entries past the
+// row's length are padding (column 0 of the range, value 0) and multiply 0,
+// not x, so that an infinity or NaN of x they do not belong to stays out of
+// the sum.
+template <int L, int MODE>
+__device__ __forceinline__ float csr_group_sum(CsrPairs<MODE>& cur, const f32x2* __restrict__ val,
+                                               const char* __restrict__ col, int pairs, int len, int t, int lane,
+                                               const float* xg) {
+    float acc = 0.f;
+    int left = len - 2 * t;  // entries of the row from this lane's first on
+    for (int p = 0; p < pairs; p += kCsrPairs) {
+        if (p) cur.load(val, col, p, pairs, lane);
+        float xa[kCsrPairs], xb[kCsrPairs];
+#pragma unroll
+        for (int u = 0; u < kCsrPairs; ++u)
+            if (p + u < pairs) {
+                if constexpr (MODE == kCsrWide) {
+                    xa[u] = xg[cur.c[u].x];
+                    xb[u] = xg[cur.c[u].y];
+                } else {
+                    xa[u] = xg[cur.c[u] & 0xffffu];
+                    xb[u] = xg[cur.c[u] >> 16];
+                }
+            }
+#pragma unroll
+        for (int u = 0; u < kCsrPairs; ++u)
+            if (p + u < pairs) {
+                acc = fmaf(cur.v[u].x, left > 0 ? xa[u] : 0.f, acc);
+                acc = fmaf(cur.v[u].y, left > 1 ? xb[u] : 0.f, acc);
+                left -= 2 * L;
+            }
+    }
+    return acc;
+}
+
+// L lanes per row.  A workgroup of kCsrThreads threads owns one row group:
+// kCsrThreads / L rows of at most 64 entries, the longest first, so that the
+// 64 / L rows of a wave have nearly equal lengths; the wave's entries are
+// stored pair by pair, 64 lanes side by side (8 + 4 bytes per lane and pair
+// when the group's columns span at most 65536, else 8 + 8).  The x range of
+// the group is staged in LDS when it fits (kCsrWindow).
+// Bound by HBM on large matrices with columns near the diagonal: 1,000,003
+// rows of 9..27 entries within ~2000 columns (159 MB by CSR's count, 126 MB
+// stored) take 26.0 us, 6.1 TB/s of CSR bytes.  Waves that staged 512
+// consecutive entries' products in LDS and summed each row from there took
+// 80 us: one L1 line per gathered x (an LDS read of the staged range is
+// several times cheaper) and a chain of block descriptor, columns, x, row
+// pointer and row sum in every wave.  512 threads per workgroup measured
+// level with 1024 and 3 % ahead of 256 (the same matrix and 57 others); 4
+// pairs in flight 2 % ahead of 2 and level with 8.
+template <int L>
+__global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptive m, int nlong_wg,
+                                                                   const float* __restrict__ x,
+                                                                   float* __restrict__ y) {
+    extern __shared__ float xs[];
     const int lane = threadIdx.x & 63;
-    const int b = blockIdx.x * 4 + wid;
-    if (b >= nblocks) return;
-    const int4 blk = blocks[b];
-    const int r0 = blk.x, tag = blk.y, n0 = blk.z, n1 = blk.w;
-    if (tag < 0 || tag - r0 == 1) {
-        // VECTOR (one row) or LONG (one chunk of a long row).
-        float acc = 0.f;
-        int k = n0 + lane;
-        for (; k + 192 < n1; k += 256) {
-            int c0 = ld_stream(col + k), c1 = ld_stream(col + k + 64), c2 = ld_stream(col + k + 128),
-                c3 = ld_stream(col + k + 192);
-            float v0 = ld_stream(val + k), v1 = ld_stream(val + k + 64), v2 = ld_stream(val + k + 128),
-                  v3 = ld_stream(val + k + 192);
-            acc = fmaf(v0, x[c0], acc);
-            acc = fmaf(v1, x[c1], acc);
-            acc = fmaf(v2, x[c2], acc);
-            acc = fmaf(v3, x[c3], acc);
-        }
-        for (; k < n1; k += 64) acc = fmaf(ld_stream(val + k), x[ld_stream(col + k)], acc);
-        acc = wave_sum(acc);
-        if (lane == 0) {
-            if (tag < 0)
-                carry[-tag - 1] = (double)acc;
-            else if (n1 > n0)
-                y[r0] += acc;
-        }
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    if ((int)blockIdx.x < nlong_wg) {
+        const int b = blockIdx.x * kCsrWaves + wave;
+        if (b < m.nblocks) csr_long_block(m, b, x, y, lane);
         return;
     }
-    // STREAM: rows [r0, tag), nnz [n0, n1), n1 - n0 <= 512.
-    const int n = n1 - n0;
-    float* sh = lds[wid];
-#pragma unroll
-    for (int u = 0; u < kCsrStreamPerLane; ++u) {
-        const int k = lane + 64 * u;
-        if (k < n) sh[k] = ld_stream(val + n0 + k) * x[ld_stream(col + n0 + k)];
-    }
-    wave_lds_sync();
-    const int r = r0 + lane;
-    if (r < tag) {
-        const int s = rp[r] - n0, e = rp[r + 1] - n0;
-        if (e > s) {
-            float acc = 0.f;
-            for (int k = s; k < e; ++k) acc += sh[k];
-            y[r] += acc;
+    const int g = xcd_tile(blockIdx.x - nlong_wg, m.ngroups);
+    const CsrGroup d = m.groups[g];
+    const int p0 = m.pair[g * kCsrWaves + wave], pairs = m.pair[g * kCsrWaves + wave + 1] - p0;
+    const int t = threadIdx.x % L;
+    const unsigned meta = m.lane[g * (kCsrThreads / L) + threadIdx.x / L];  // length << 16 | row in group
+    const int len = (int)(meta >> 16);
+    float* yp = y + d.row0 + (meta & 0xffffu);
+    const bool out = t == 0 && len > 0;
+    const float yo = out ? *yp : 0.f;
+    const f32x2* val = reinterpret_cast<const f32x2*>(m.gval) + (size_t)p0 * 64;
+    const char* col = reinterpret_cast<const char*>(m.gcol) +
+                      ((size_t)d.col256 + (size_t)(p0 - d.pair0) * (d.mode == kCsrWide ? 2 : 1)) * 256;
+    float acc;
+    if (d.mode == kCsrStaged) {
+        CsrPairs<kCsrStaged> first;
+        first.load(val, col, 0, pairs, lane);  // in flight while x is staged
+        const float* src = x + d.x0;
+        for (int i = threadIdx.x * 4; i < d.xn; i += kCsrThreads * 4) {
+            if (i + 4 <= d.xn) {
+                const f32x4a4 q = *reinterpret_cast<const f32x4a4*>(src + i);
+                *reinterpret_cast<float4*>(xs + i) = make_float4(q.x, q.y, q.z, q.w);
+            } else {
+                for (int j = i; j < d.xn; ++j) xs[j] = src[j];
+            }
         }
+        __syncthreads();
+        acc = csr_group_sum<L, kCsrStaged>(first, val, col, pairs, len, t, lane, xs);
+    } else if (d.mode == kCsrNear) {
+        CsrPairs<kCsrNear> first;
+        first.load(val, col, 0, pairs, lane);
+        acc = csr_group_sum<L, kCsrNear>(first, val, col, pairs, len, t, lane, x + d.x0);
+    } else {
+        CsrPairs<kCsrWide> first;
+        first.load(val, col, 0, pairs, lane);
+        acc = csr_group_sum<L, kCsrWide>(first, val, col, pairs, len, t, lane, x);
     }
+    acc = group_sum<L>(acc);
+    if (out) *yp = yo + acc;
 }
 
 // One column slice of the column-sliced CSR.  Same block kinds as
@@ -219,10 +318,23 @@ int launch_csr_vector(const DevCsr& m, int lanes, const float* x, float* y, hipS
     return (int)hipGetLastError();
 }
 
+template <int L>
+static void csr_adaptive_launch(const DevCsrAdaptive& m, const float* x, float* y, hipStream_t st) {
+    const int nlong_wg = (m.nblocks + kCsrWaves - 1) / kCsrWaves;
+    hipLaunchKernelGGL(dev::csr_adaptive_kernel<L>, dim3(nlong_wg + m.ngroups), dim3(kCsrThreads),
+                       (size_t)m.lds_floats * 4, st, m, nlong_wg, x, y);
+}
+
 int launch_csr_adaptive(const DevCsrAdaptive& m, const float* x, float* y, hipStream_t st) {
-    if (m.nblocks > 0) {
-        hipLaunchKernelGGL(dev::csr_adaptive_kernel, dim3((m.nblocks + 3) / 4), dim3(256), 0, st, m.csr.row_ptr,
-                           m.csr.col, m.csr.val, m.blocks, m.nblocks, x, y, m.carry);
+    if (m.nblocks > 0 || m.ngroups > 0) {
+        switch (m.lanes) {
+            case 1: csr_adaptive_launch<1>(m, x, y, st); break;
+            case 2: csr_adaptive_launch<2>(m, x, y, st); break;
+            case 4: csr_adaptive_launch<4>(m, x, y, st); break;
+            case 8: csr_adaptive_launch<8>(m, x, y, st); break;
+            case 16: csr_adaptive_launch<16>(m, x, y, st); break;
+            default: return (int)hipErrorInvalidValue;
+        }
         int e = (int)hipGetLastError();
         if (e) return e;
     }

@@ -12,6 +12,7 @@
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -131,9 +132,10 @@ int pow2_floor(int v) {
 }
 
 bool cols_ok(const int* c, size_t n, int lo, int hi) {
-    for (size_t i = 0; i < n; ++i)
-        if (c[i] < lo || c[i] >= hi) return false;
-    return true;
+    bool ok = true;
+#pragma omp parallel for schedule(static) num_threads(omp_threads()) reduction(&& : ok) if (n > 65536)
+    for (long long i = 0; i < (long long)n; ++i) ok = ok && c[i] >= lo && c[i] < hi;
+    return ok;
 }
 
 template <class F>
@@ -587,9 +589,9 @@ static int validate_csr(const clspmv_csr_matrix* m) {
     return CLSPMV_OK;
 }
 
+// Uploads the arrays of a validated CSR matrix as they are.
 static int upload_csr(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_csr_matrix* m) {
-    int rc = validate_csr(m);
-    if (rc) return rc;
+    int rc = CLSPMV_OK;
     const int rows = m->matinfo.height;
     const size_t nnz = (size_t)m->csr_row_ptr[rows];
     p->csr.row_ptr = (const int*)p->add(ctx, m->csr_row_ptr, ((size_t)rows + 1) * 4, &rc);
@@ -726,6 +728,189 @@ int build_csr_sliced(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const int
     d.n_long = (int)long_rows.size();
     p->csrs = d;
     p->carry_bytes = (long long)std::max(1, slots) * 8;
+    return CLSPMV_OK;
+}
+
+// Lanes per row of the row groups: more of them while the rows alone give
+// fewer than kCsrFillWaves wavefronts (eight per CU) and a row still feeds
+// its lanes a pair each (8000 rows of 20..60 entries: 3.3 us, 8.0 with the
+// 512-entry waves that this layout replaced).
+constexpr long long kCsrFillWaves = 2048;
+int csr_group_lanes(long long rows, long long nnz) {
+    int lanes = 1;
+    while (lanes < 16 && rows * lanes < 64 * kCsrFillWaves && nnz >= rows * 4 * lanes) lanes *= 2;
+    return lanes;
+}
+
+// Staging reads the group's whole x range, coalesced; reading x from memory
+// costs up to one cache line per entry.  Staging is taken up to this many
+// columns per entry: 1M rows of 1..4 entries with 3 columns per entry ran
+// 8.6 us unstaged and 9.3 staged, of 2..7 entries with 1.3 columns per entry
+// 12.4 unstaged and 10.9 staged; small matrices did not care.
+constexpr long long kCsrStagePays = 2;
+
+// Builds the adaptive layout (DevCsrAdaptive) from CSR arrays (any column
+// order within a row).  Row groups take the rows of 1..kCsrStreamMaxRowLen
+// entries in order, kCsrThreads / lanes of them each (fewer where their
+// distance would not fit 16 bits), the longest first within the group;
+// longer rows become VECTOR / LONG blocks over compacted arrays.
+int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const int* ci, const float* cv, int rows) {
+    auto len = [&](int r) { return rp[r + 1] - rp[r]; };
+    long long short_rows = 0, short_nnz = 0;
+    std::vector<int> long_list;  // rows longer than kCsrStreamMaxRowLen
+    for (int r = 0; r < rows; ++r) {
+        const int l = len(r);
+        if (l > kCsrStreamMaxRowLen) {
+            long_list.push_back(r);
+        } else {
+            short_rows += l > 0;
+            short_nnz += l;
+        }
+    }
+    const int lanes = csr_group_lanes(short_rows, short_nnz);
+    const int cap = kCsrThreads / lanes, wave_rows = 64 / lanes;
+    // rows [begin[g], begin[g + 1]) of group g (rows outside it are skipped)
+    std::vector<int> begin;
+    for (int r = 0, n = 0, row0 = 0; r < rows; ++r) {
+        const int l = len(r);
+        if (l == 0 || l > kCsrStreamMaxRowLen) continue;
+        if (begin.empty() || n == cap || r - row0 > 0xffff) {
+            begin.push_back(r);
+            row0 = r;
+            n = 0;
+        }
+        ++n;
+    }
+    const int ng = (int)begin.size();
+    begin.push_back(rows);
+    std::vector<CsrGroup> groups((size_t)ng);
+    std::vector<unsigned> lane((size_t)std::max(1, ng) * cap, 0u);
+    std::vector<int> pair((size_t)ng * kCsrWaves + 1, 0);  // pairs of each wave, then their prefix
+#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) if (ng > 16)
+    for (int g = 0; g < ng; ++g) {
+        // counting sort by length, longest first, rows of one length in order
+        int at[kCsrStreamMaxRowLen + 2] = {0};
+        int lo = INT32_MAX, hi = 0;
+        long long gn = 0;
+        for (int r = begin[(size_t)g]; r < begin[(size_t)g + 1]; ++r) {
+            const int l = len(r);
+            if (l == 0 || l > kCsrStreamMaxRowLen) continue;
+            at[kCsrStreamMaxRowLen - l + 1]++;
+            gn += l;
+            for (int k = rp[r]; k < rp[r + 1]; ++k) {
+                lo = std::min(lo, ci[k]);
+                hi = std::max(hi, ci[k]);
+            }
+        }
+        for (int i = 0; i <= kCsrStreamMaxRowLen; ++i) at[i + 1] += at[i];
+        unsigned* slot = &lane[(size_t)g * cap];
+        const int row0 = begin[(size_t)g];
+        for (int r = row0; r < begin[(size_t)g + 1]; ++r) {
+            const int l = len(r);
+            if (l == 0 || l > kCsrStreamMaxRowLen) continue;
+            slot[at[kCsrStreamMaxRowLen - l]++] = (unsigned)l << 16 | (unsigned)(r - row0);
+        }
+        for (int w = 0; w < kCsrWaves; ++w)
+            pair[(size_t)g * kCsrWaves + w + 1] = ((int)(slot[w * wave_rows] >> 16) + 2 * lanes - 1) / (2 * lanes);
+        CsrGroup& d = groups[(size_t)g];
+        d.row0 = row0;
+        d.x0 = lo & ~3;  // staged in 16-byte loads
+        d.xn = hi - d.x0 + 1;
+        d.mode = d.xn <= kCsrWindow && d.xn <= kCsrStagePays * gn ? kCsrStaged : d.xn <= 65536 ? kCsrNear : kCsrWide;
+    }
+    long long pairs = 0, col256 = 0;
+    int lds_floats = 0;
+    for (int g = 0; g < ng; ++g) {
+        groups[(size_t)g].pair0 = (int)pairs;
+        groups[(size_t)g].col256 = (int)col256;
+        const long long p0 = pairs;
+        for (int w = 0; w < kCsrWaves; ++w) {
+            pairs += pair[(size_t)g * kCsrWaves + w + 1];
+            pair[(size_t)g * kCsrWaves + w + 1] = (int)pairs;
+        }
+        col256 += (pairs - p0) * (groups[(size_t)g].mode == kCsrWide ? 2 : 1);
+        if (groups[(size_t)g].mode == kCsrStaged) lds_floats = std::max(lds_floats, (groups[(size_t)g].xn + 3) & ~3);
+        if (col256 > INT32_MAX) return CLSPMV_E_TOO_LARGE;
+    }
+    std::unique_ptr<float[]> gval(new (std::nothrow) float[std::max<size_t>(1, (size_t)pairs * 128)]);
+    std::unique_ptr<char[]> gcol(new (std::nothrow) char[std::max<size_t>(1, (size_t)col256 * 256)]);
+    if (!gval || !gcol) return CLSPMV_E_NOMEM;
+#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) if (ng > 16)
+    for (int g = 0; g < ng; ++g) {
+        const CsrGroup& d = groups[(size_t)g];
+        const bool wide = d.mode == kCsrWide;
+        const int g0 = d.pair0, g1 = pair[(size_t)(g + 1) * kCsrWaves];
+        char* col = gcol.get() + (size_t)d.col256 * 256;
+        std::memset(gval.get() + (size_t)g0 * 128, 0, (size_t)(g1 - g0) * 512);
+        std::memset(col, 0, (size_t)(g1 - g0) * (wide ? 512 : 256));  // padding: column 0 (wide) or x0
+        for (int i = 0; i < cap; ++i) {
+            const unsigned meta = lane[(size_t)g * cap + i];
+            const int l = (int)(meta >> 16);
+            const int k0 = l ? rp[d.row0 + (int)(meta & 0xffffu)] : 0;
+            const size_t p0 = (size_t)pair[(size_t)g * kCsrWaves + i / wave_rows];
+            for (int j = 0; j < l; ++j) {
+                const size_t q = ((p0 + j / (2 * lanes)) * 64 + (i % wave_rows) * lanes + (j / 2) % lanes) * 2 + j % 2;
+                gval[q] = cv[k0 + j];
+                if (wide)
+                    reinterpret_cast<int*>(col)[q - (size_t)g0 * 128] = ci[k0 + j];
+                else
+                    reinterpret_cast<uint16_t*>(col)[q - (size_t)g0 * 128] = (uint16_t)(ci[k0 + j] - d.x0);
+            }
+        }
+    }
+    // the long rows' blocks, over their entries only
+    std::vector<int4> blocks;
+    std::vector<int> long_rows, long_first{0}, long_at;
+    int slots = 0, long_nnz = 0;
+    for (int r : long_list) {
+        const int n0 = long_nnz, n1 = n0 + len(r);
+        long_at.push_back(n0);
+        long_nnz = n1;
+        if (len(r) <= kCsrLongChunk) {
+            blocks.push_back(make_int4(r, r + 1, n0, n1));
+            continue;
+        }
+        long_rows.push_back(r);
+        for (int a = n0; a < n1; a += kCsrLongChunk) {
+            blocks.push_back(make_int4(r, -(slots + 1), a, std::min(n1, a + kCsrLongChunk)));
+            ++slots;
+        }
+        long_first.push_back(slots);
+    }
+    std::unique_ptr<int[]> lcol(new (std::nothrow) int[(size_t)std::max(1, long_nnz)]);
+    std::unique_ptr<float[]> lval(new (std::nothrow) float[(size_t)std::max(1, long_nnz)]);
+    if (!lcol || !lval) return CLSPMV_E_NOMEM;
+#pragma omp parallel for schedule(dynamic, 16) num_threads(omp_threads()) if (long_nnz > 65536)
+    for (long long i = 0; i < (long long)long_list.size(); ++i) {
+        const int r = long_list[(size_t)i];
+        std::copy(ci + rp[r], ci + rp[r + 1], lcol.get() + long_at[(size_t)i]);
+        std::copy(cv + rp[r], cv + rp[r + 1], lval.get() + long_at[(size_t)i]);
+    }
+    DevCsrAdaptive d{};
+    int rc = 0;
+    auto up = [&](const void* h, size_t bytes) -> const void* {
+        return rc ? nullptr : p->add(ctx, h, bytes, &rc);
+    };
+    d.groups = (const CsrGroup*)up(groups.data(), groups.size() * sizeof(CsrGroup));
+    d.pair = (const int*)up(pair.data(), pair.size() * 4);
+    d.lane = (const unsigned*)up(lane.data(), lane.size() * 4);
+    d.gval = (const float*)up(gval.get(), (size_t)pairs * 512);
+    d.gcol = up(gcol.get(), (size_t)col256 * 256);
+    d.col = (const int*)up(lcol.get(), (size_t)long_nnz * 4);
+    d.val = (const float*)up(lval.get(), (size_t)long_nnz * 4);
+    d.blocks = (const int4*)up(blocks.data(), blocks.size() * sizeof(int4));
+    d.long_rows = (const int*)up(long_rows.data(), long_rows.size() * 4);
+    d.long_first = (const int*)up(long_first.data(), long_first.size() * 4);
+    if (rc) return rc;
+    p->carry_bytes = (long long)std::max(1, slots) * 8;
+    d.carry = (double*)p->scratch((size_t)p->carry_bytes, &rc);
+    if (rc) return rc;
+    d.ngroups = ng;
+    d.lanes = lanes;
+    d.lds_floats = lds_floats;
+    d.nblocks = (int)blocks.size();
+    d.n_long = (int)long_rows.size();
+    p->csra = d;
     return CLSPMV_OK;
 }
 
@@ -1287,7 +1472,8 @@ extern "C" {
 
 int clspmv_part_csr_scalar(clspmv_ctx_t ctx, const clspmv_csr_matrix* m, int method, clspmv_part_t* out) {
     return make_part(ctx, out, [&](clspmv_part_t p) {
-        int rc = upload_csr(ctx, p, m);
+        int rc = validate_csr(m);
+        if (!rc) rc = upload_csr(ctx, p, m);
         if (rc) return rc;
         fill_info(p, CLSPMV_FMT_CSR_SCALAR, 0, m->matinfo.height, m->matinfo.width, m->matinfo.nnz, "csr_scalar", 1);
         (void)method;
@@ -1296,10 +1482,10 @@ int clspmv_part_csr_scalar(clspmv_ctx_t ctx, const clspmv_csr_matrix* m, int met
 }
 
 // method 0: L lanes per row (L from the mean row length);
-// method 1: adaptive row blocks (stream / vector / long-row split).
+// method 1: adaptive (row groups / vector / long-row split).
 int clspmv_part_csr_vector(clspmv_ctx_t ctx, const clspmv_csr_matrix* m, int method, clspmv_part_t* out) {
     return make_part(ctx, out, [&](clspmv_part_t p) {
-        int rc = upload_csr(ctx, p, m);
+        int rc = validate_csr(m);
         if (rc) return rc;
         const int rows = m->matinfo.height;
         const int* rp = m->csr_row_ptr;
@@ -1307,23 +1493,16 @@ int clspmv_part_csr_vector(clspmv_ctx_t ctx, const clspmv_csr_matrix* m, int met
         if (method == kMethodXtile) {
             rc = build_xtile(ctx, p, m->csr_row_ptr, m->csr_col_id, m->csr_data, rows, m->matinfo.width);
             if (rc) return rc;
-            for (int i = 0; i < 3; ++i) p->bufs[i].release();  // plain CSR upload unused
             return finish_xtile(p, CLSPMV_FMT_CSR_VECTOR, rows, m->matinfo.width, m->matinfo.nnz);
         }
         if (method == 2) {
             rc = build_csr_sliced(ctx, p, m->csr_row_ptr, m->csr_col_id, m->csr_data, rows, m->matinfo.width);
             if (rc) return rc;
-            // the plain CSR upload is not used by this layout
-            for (int i = 0; i < 3; ++i) p->bufs[i].release();
-            char name[32];
-            std::snprintf(name, sizeof(name), "csr_sliced_S%d", p->csrs.nslices);
-            fill_info(p, CLSPMV_FMT_CSR_VECTOR, 2, rows, m->matinfo.width, m->matinfo.nnz, name,
-                      p->csrs.nslices + (p->csrs.n_long ? 1 : 0));
-            p->info.stored_bytes -= p->carry_bytes;
-            p->info.alg_bytes -= p->carry_bytes;
-            return CLSPMV_OK;
+            return finish_sliced(p, CLSPMV_FMT_CSR_VECTOR, rows, m->matinfo.width, m->matinfo.nnz, "csr");
         }
         if (method == 0) {
+            rc = upload_csr(ctx, p, m);
+            if (rc) return rc;
             double mean = rows ? (double)nnz / rows : 0.0;
             p->csr_lanes = std::min(64, std::max(2, pow2_floor((int)(mean / 2.0 + 0.5))));
             char name[32];
@@ -1331,53 +1510,13 @@ int clspmv_part_csr_vector(clspmv_ctx_t ctx, const clspmv_csr_matrix* m, int met
             fill_info(p, CLSPMV_FMT_CSR_VECTOR, 0, rows, m->matinfo.width, m->matinfo.nnz, name, 1);
             return CLSPMV_OK;
         }
-        std::vector<int4> blocks;
-        std::vector<int> long_rows, long_first{0};
-        int slots = 0;
-        int r = 0;
-        while (r < rows) {
-            const int len = rp[r + 1] - rp[r];
-            if (len > kCsrStreamMaxRowLen) {
-                if (len <= kCsrLongChunk) {
-                    blocks.push_back(make_int4(r, r + 1, rp[r], rp[r + 1]));
-                } else {
-                    long_rows.push_back(r);
-                    for (int n0 = rp[r]; n0 < rp[r + 1]; n0 += kCsrLongChunk) {
-                        int n1 = std::min(rp[r + 1], n0 + kCsrLongChunk);
-                        blocks.push_back(make_int4(r, -(slots + 1), n0, n1));
-                        ++slots;
-                    }
-                    long_first.push_back(slots);
-                }
-                ++r;
-                continue;
-            }
-            const int r0 = r;
-            int n = 0;
-            while (r < rows && r - r0 < 64) {
-                const int l = rp[r + 1] - rp[r];
-                if (l > kCsrStreamMaxRowLen || n + l > kCsrStreamMaxNnz) break;
-                n += l;
-                ++r;
-            }
-            blocks.push_back(make_int4(r0, r, rp[r0], rp[r]));
-        }
-        p->csra.csr = p->csr;
-        p->csra.nblocks = (int)blocks.size();
-        p->csra.blocks = (const int4*)p->add(ctx, blocks.data(), blocks.size() * sizeof(int4), &rc);
-        if (rc) return rc;
-        p->csra.n_long = (int)long_rows.size();
-        p->csra.carry = (double*)p->scratch((size_t)std::max(1, slots) * sizeof(double), &rc);
-        if (rc) return rc;
-        p->csra.long_rows = (const int*)p->add(ctx, long_rows.data(), long_rows.size() * 4, &rc);
-        if (rc) return rc;
-        p->csra.long_first = (const int*)p->add(ctx, long_first.data(), long_first.size() * 4, &rc);
+        rc = build_csr_adaptive(ctx, p, rp, m->csr_col_id, m->csr_data, rows);
         if (rc) return rc;
         fill_info(p, CLSPMV_FMT_CSR_VECTOR, 1, rows, m->matinfo.width, m->matinfo.nnz, "csr_adaptive",
                   p->csra.n_long ? 2 : 1);
         // the carry buffer is scratch, not format storage
-        p->info.stored_bytes -= (long long)std::max(1, slots) * 8;
-        p->info.alg_bytes -= (long long)std::max(1, slots) * 8;
+        p->info.stored_bytes -= p->carry_bytes;
+        p->info.alg_bytes -= p->carry_bytes;
         return CLSPMV_OK;
     });
 }
