@@ -197,7 +197,9 @@ __global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptiv
                 const f32x4a4 q = *reinterpret_cast<const f32x4a4*>(src + i);
                 *reinterpret_cast<float4*>(xs + i) = make_float4(q.x, q.y, q.z, q.w);
             } else {
-                for (int j = i; j < d.xn; ++j) xs[j] = src[j];
+#pragma unroll
+                for (int j = 0; j < 3; ++j)
+                    if (i + j < d.xn) xs[i + j] = src[i + j];
             }
         }
         __syncthreads();

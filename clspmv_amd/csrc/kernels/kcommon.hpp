@@ -107,6 +107,54 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// Lane l receives v of lane l - 1 (lane 0 keeps its own): the DPP
+// shift-the-whole-wave-right-by-one mode (control 0x138) of GFX9-family
+// parts, a VALU move instead of a trip through the LDS crossbar.
+__device__ __forceinline__ int lane_up1(int v) { return __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false); }
+__device__ __forceinline__ float lane_up1(float v) { return __int_as_float(lane_up1(__float_as_int(v))); }
+
+// v of another lane by a DPP mode of GFX9-family parts: CTRL 0x110 + d is
+// "the lane d below in the same 16-lane row", 0x142 / 0x143 broadcast lane
+// 15 / 31 into the next row(s); ROWS selects the rows written (the others,
+// and lanes with no source, read 0).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xf, false); }
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_f(float v) { return __int_as_float(dpp_i<CTRL, ROWS>(__float_as_int(v))); }
+
+// One step of a segmented inclusive scan: a lane with no segment start in
+// its range so far takes the range below (value added, start flag taken).
+__device__ __forceinline__ void seg_step(bool valid, float up_v, int up_f, float& v, int& f) {
+    const bool take = valid && !f;
+    v = take ? v + up_v : v;
+    f = take ? up_f : f;
+}
+
+// Smallest v of the 64 lanes, wave-uniform (every lane active): the row and
+// broadcast DPP moves of GFX9-family parts leave it in lane 63.
+__device__ __forceinline__ int wave_min(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xf, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xa, 0xf, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Sum over the 64 lanes as wave_min does it, wave-uniform (every lane
+// active): VALU moves only, where wave_sum's shuffles go through the LDS
+// crossbar.
+__device__ __forceinline__ float wave_total(float v) {
+    v += dpp_f<0x111, 0xf>(v);
+    v += dpp_f<0x112, 0xf>(v);
+    v += dpp_f<0x114, 0xf>(v);
+    v += dpp_f<0x118, 0xf>(v);
+    v += dpp_f<0x142, 0xa>(v);
+    v += dpp_f<0x143, 0xc>(v);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
 // Orders LDS traffic among the lanes of one wavefront (no workgroup barrier:
 // the waves of a workgroup may be on different code paths).
 __device__ __forceinline__ void wave_lds_sync() {

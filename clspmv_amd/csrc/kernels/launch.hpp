@@ -80,11 +80,10 @@ struct DevCoo {
     const int* row;
     const int* col;
     const float* val;
-    int nnz_padded;           // multiple of the chunk size
-    int nnz;                  // entries the arrays hold (nnz_padded, or fewer: the last chunk is padded on the fly)
+    int nnz;                  // the last chunk is padded as it is loaded
     int chunks;
     int rows;
-    int* carry_row;           // 2 per chunk
+    int* carry_row;           // 2 per chunk; null when no row reaches past a chunk's end by more than kCooReach
     double* carry_val;        // 2 per chunk
 };
 struct DevDia {
@@ -261,5 +260,14 @@ constexpr int kCsrStreamMaxRowLen = 64;                 // longer rows get their
 constexpr int kCsrLongChunk = 1024;
 constexpr int kCooPerLane = 8;
 constexpr int kCooChunk = 64 * kCooPerLane;             // 512 nnz per wave
+// Entries of the next chunk from which a chunk finishes its last row: one
+// per lane of its wave.
+constexpr int kCooReach = 64;
+// A workgroup of T threads stages at most this many columns of x in LDS:
+// with its segments' rows 20 or 40 KiB, 32 waves per CU.
+constexpr int coo_window(int threads) { return threads == 256 ? 3040 : 6080; }
+// Up to this many chunks 256 threads per workgroup: more CUs take part (up
+// to 0.5 us less); beyond, 512 threads share a wider x range.
+constexpr int kCooFewChunks = 2048;
 
 }  // namespace clspmv

@@ -1568,16 +1568,22 @@ int clspmv_part_coo(clspmv_ctx_t ctx, const clspmv_coo_matrix* m, int method, cl
         if (rc) return rc;
         p->coo.val = (const float*)p->add(ctx, vv.data(), padded * 4, &rc);
         if (rc) return rc;
-        p->coo.nnz_padded = (int)padded;
-        p->coo.nnz = (int)padded;
+        p->coo.nnz = nnz;
         p->coo.chunks = chunks;
         p->coo.rows = rows;
-        const size_t ncarry = (size_t)std::max(1, 2 * chunks);
-        p->coo.carry_row = (int*)p->scratch(ncarry * 4, &rc);
-        if (rc) return rc;
-        p->coo.carry_val = (double*)p->scratch(ncarry * 8, &rc);
-        if (rc) return rc;
-        fill_info(p, CLSPMV_FMT_COO, 0, rows, cols, nnz, "coo_segment", 2);
+        // carries are needed where a row goes on past a chunk's end for more
+        // than kCooReach entries
+        bool carries = false;
+        for (long long k = kCooChunk; k + kCooReach < nnz && !carries; k += kCooChunk)
+            carries = m->coo_row_id[k - 1] == m->coo_row_id[k + kCooReach];
+        const size_t ncarry = carries ? 2 * (size_t)chunks : 0;
+        if (carries) {
+            p->coo.carry_row = (int*)p->scratch(ncarry * 4, &rc);
+            if (rc) return rc;
+            p->coo.carry_val = (double*)p->scratch(ncarry * 8, &rc);
+            if (rc) return rc;
+        }
+        fill_info(p, CLSPMV_FMT_COO, 0, rows, cols, nnz, "coo_segment", carries ? 2 : 1);
         p->info.stored_bytes -= (long long)ncarry * 12;
         p->info.alg_bytes -= (long long)ncarry * 12;
         (void)method;
@@ -2080,7 +2086,6 @@ int clspmv_coo_spmv_noalloc(clspmv_ctx_t ctx, int rows, int nnz, const int* d_ro
     m.col = d_col;
     m.val = d_val;
     m.chunks = (nnz + kCooChunk - 1) / kCooChunk;
-    m.nnz_padded = m.chunks * kCooChunk;
     m.nnz = nnz;
     m.rows = rows;
     // every carry slot of the m.chunks chunks is written by the segment
