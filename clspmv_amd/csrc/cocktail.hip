@@ -39,6 +39,10 @@ struct clspmv_gpumat_s {
     // every part covers rows of its own (row runs of the plan): parts may
     // then run side by side on the extra streams below
     bool disjoint = false;
+    // iterations per launch of a matrix that is one narrow-band DIA part (0:
+    // other matrices) and the two vectors its launches alternate between
+    int step_limit = 0;
+    DevBuf step[2];
     std::vector<hipStream_t> aux;  // created on first concurrent call
     std::vector<hipEvent_t> ev;    // ev[0]: fork; ev[1 + a]: join of aux[a]
     ~clspmv_gpumat_s() {
@@ -49,6 +53,7 @@ struct clspmv_gpumat_s {
         for (auto p : parts) clspmv_part_free(p);
         x.release();
         y.release();
+        for (auto& b : step) b.release();
     }
 };
 
@@ -169,12 +174,32 @@ int enqueue_concurrent(clspmv_gpumat_s* g, int passes, hipStream_t st) {
     return e == hipSuccess ? CLSPMV_OK : hip_status(e, "join");
 }
 
+// `iterations` (>= 2) iterations {y += A x; x := y}, several per launch: the
+// first launch reads x and y, the last writes both, those between alternate
+// between the object's two step vectors.
+int enqueue_steps(clspmv_gpumat_s* g, int iterations, hipStream_t st) {
+    const int launches = std::max(2, (iterations + g->step_limit - 1) / g->step_limit);
+    float *x = (float*)g->x.ptr, *y = (float*)g->y.ptr;
+    const float *xi = x, *yi = y;
+    for (int i = 0, done = 0; i < launches; ++i) {
+        const int steps = (iterations - done) / (launches - i);
+        const bool last = i == launches - 1;
+        float* yo = last ? y : (float*)g->step[i & 1].ptr;
+        const int e = clspmv_part_launch_steps(g->parts[0], steps, xi, yi, last ? x : nullptr, yo, st);
+        if (e) return hip_status((hipError_t)e, "iteration launch");
+        xi = yi = yo;
+        done += steps;
+    }
+    return CLSPMV_OK;
+}
+
 // ntimes passes on the context stream: whole graphs of kGraphPasses passes,
 // then one graph of the remainder.
 int run_passes(clspmv_gpumat_s* g, int ntimes, bool iterate) {
     hipStream_t st = g->ctx->stream();
     if (!g_use_graph && !iterate && g_streams && g->disjoint && g->parts.size() > 1 && ntimes > 0)
         return enqueue_concurrent(g, ntimes, st);
+    if (!g_use_graph && iterate && g->step_limit > 0 && ntimes > 1) return enqueue_steps(g, ntimes, st);
     if (!g_use_graph || g->parts.empty()) return enqueue_passes(g, ntimes, iterate, st);
     for (int done = 0; done < ntimes;) {
         const int n = std::min(kGraphPasses, ntimes - done);
@@ -893,6 +918,15 @@ int init_from_plan(clspmv_ctx_t ctx, const clspmv_plan_s* P, const float* vec, c
     if (!rc) {
         g->disjoint = !P->parts.empty();
         for (const PlanPart& q : P->parts) g->disjoint = g->disjoint && q.source == 9;
+        // here and not at the first call: that may be under stream capture
+        if (g->parts.size() == 1 && g->row0[0] == 0 && g->width == g->height) {
+            clspmv_part_info inf;
+            clspmv_part_get_info(g->parts[0], &inf);
+            if (inf.rows == g->height && inf.cols == g->width) g->step_limit = clspmv_part_step_limit(g->parts[0]);
+        }
+        if (g->step_limit > 0)
+            for (auto& b : g->step)
+                if (!rc) rc = b.alloc((size_t)g->height * 4);
     }
     if (!rc) rc = clspmv_synchronize(ctx);
     if (rc) {

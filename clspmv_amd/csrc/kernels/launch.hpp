@@ -92,6 +92,31 @@ struct DevDia {
     int L, ndiag, rows, cols;
     int offmin, offmax;  // smallest and largest diagonal offset
 };
+// Several iterations {y += A x; x := y} of an n x n narrow-band matrix per
+// launch (k_dia.hip: dia_steps_kernel).
+constexpr int kDiaStepThreads = 1024;
+constexpr int kDiaStepDiags = 8;       // diagonals at most (in registers, per row slot)
+constexpr int kDiaStepSlots = 10;      // rows per thread at most: 8 x 10 diagonal registers
+constexpr int kDiaStepFloats = 20480;  // vector range of one of the two LDS buffers: 80 KiB
+constexpr int kDiaStepGroups = 256;    // workgroups: one per CU
+inline int dia_step_reach(const DevDia& m) { return m.offmax > -m.offmin ? m.offmax : -m.offmin; }
+inline int dia_step_rows(const DevDia& m) { return (m.rows + kDiaStepGroups - 1) / kDiaStepGroups; }
+// Steps one launch takes at most (0: none).  Its range, R rows and steps * w
+// to each side, has to fit the row slots and an LDS buffer; and since a
+// launch costs a start and a read of the range's diagonals while a step costs
+// work for the whole range, the cost per step is least near 100 / sqrt(w)
+// steps: measured best at 6 for w = 256 (65,536 rows), 4 for 512 (262,144)
+// and 3 to 4 for 700 (490,000), 12 for 64.
+inline int dia_step_limit(const DevDia& m) {
+    if (m.rows != m.cols || m.rows < 1 || m.ndiag < 1 || m.ndiag > kDiaStepDiags) return 0;
+    const long long w = dia_step_reach(m), R = dia_step_rows(m);
+    const long long by_lds = (kDiaStepFloats - 2 * w) / kDiaStepThreads;
+    const long long rows = (by_lds < kDiaStepSlots ? by_lds : kDiaStepSlots) * kDiaStepThreads;
+    long long most = 64;
+    while (most > 0 && rows < m.rows && rows < R + 2 * most * w) --most;
+    while (most > 1 && most * most * w > 10000) --most;
+    return (int)most;
+}
 struct DevBdia {
     const int* bptr;
     const int* offsets;
@@ -236,6 +261,8 @@ int launch_csr_adaptive(const DevCsrAdaptive& m, const float* x, float* y, hipSt
 int launch_csr_sliced(const DevCsrSliced& m, const float* x, float* y, hipStream_t st);
 int launch_coo(const DevCoo& m, const float* x, float* y, hipStream_t st);
 int launch_dia(const DevDia& m, int method, const float* x, float* y, hipStream_t st);
+int launch_dia_steps(const DevDia& m, int method, int steps, const float* x, const float* y, float* xout, float* yout,
+                     hipStream_t st);
 int launch_bdia(const DevBdia& m, int method, const float* x, float* y, hipStream_t st);
 int launch_bell(const DevBell& m, const float* x, float* y, hipStream_t st);
 int launch_sbell(const DevSbell& m, const float* x, float* y, hipStream_t st);

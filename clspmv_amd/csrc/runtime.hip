@@ -2026,6 +2026,17 @@ int clspmv_part_launch(clspmv_part_t p, const float* x, float* y, hipStream_t st
     }
 }
 
+int clspmv_part_step_limit(clspmv_part_t p) {
+    if (p->mixed || p->info.format != CLSPMV_FMT_DIA || p->info.method > 1) return 0;
+    return dia_step_limit(p->dia);
+}
+
+int clspmv_part_launch_steps(clspmv_part_t p, int steps, const float* x, const float* y, float* xout, float* yout,
+                             hipStream_t st) {
+    if (!clspmv_part_step_limit(p)) return (int)hipErrorInvalidValue;
+    return launch_dia_steps(p->dia, p->info.method, steps, x, y, xout, yout, st);
+}
+
 int clspmv_part_spmv(clspmv_part_t p, const float* d_x, float* d_y, int ntimes) {
     if (!p || !d_x || !d_y || ntimes < 0) return CLSPMV_E_INVALID;
     if ((reinterpret_cast<uintptr_t>(d_x) | reinterpret_cast<uintptr_t>(d_y)) & 15) {

@@ -119,8 +119,10 @@ int clspmv_do_spmv(clspmv_gpumat_t gpumat, int ntimes);
 /* The iteration of the reference's example (A/src/eval.cpp:19-72, with
  * cpy_vector_from_gpu :1510-1556): `iterations` times { y += A x; x := y },
  * all enqueued on the device with no host round trip (x := y by a copy
- * kernel; from captured graphs of up to 64 iterations with
- * "cocktail_graph" 1).  Square matrices only; asynchronous. */
+ * kernel; a narrow-band matrix that is one DIA part of at most 8 diagonals
+ * takes several iterations per launch instead, the same bits; from captured
+ * graphs of up to 64 iterations with "cocktail_graph" 1).  Square matrices
+ * only; asynchronous. */
 int clspmv_power_iterate(clspmv_gpumat_t gpumat, int iterations);
 /* cpy_vector_from_cpu / _from_gpu, cpy_result_from_cpu / _from_gpu /
  * _to_cpu / _to_gpu (:1458-1588).  *_gpu take device pointers. */
