@@ -28,6 +28,14 @@
 // Waves take items i, i + W, i + 2W, ... (W = waves in the grid), so the
 // launch is one grid whatever the number of matrices.  No atomics: results
 // are deterministic.
+// Bound by gathering X: from L2 while a matrix's X fits there, else from the
+// Infinity Cache (2^18 rows x 32 scattered entries, k = 16: 4.6 TB/s of X
+// rows).  Item and matrix descriptors are wave-uniform and live in scalar
+// registers: 62 vector registers instead of 90, 8 waves per SIMD instead of
+// 5 (27-point stencils of 2^18 rows, k = 1 / 4 / 16: 45 / 50 / 95 -> 31 / 34
+// / 68 us; 3 x 3 blocks alike).  Items dealt to the XCDs in runs of 4 to 512
+// neighbours, streaming hints on the entries and shorter LONG chunks were
+// all measured level or slower.
 #include "kcommon.hpp"
 #include "launch.hpp"
 
@@ -100,27 +108,61 @@ __device__ void spmm_stream(const SpmmMat& m, int r0, int r1, int* s_col, float*
     const int lpr = Ln::V * split, slots = 64 / lpr;
     const int slot = lane / lpr, sp = (lane / Ln::V) % split, v = lane % Ln::V;
     const float* xb = m.x + v * Ln::W;
-    for (int r = r0 + slot; r < r1; r += slots) {
-        const int a = m.row_ptr[r] - n0, b = m.row_ptr[r + 1] - n0;
-        Vec<Ln::W> acc;
-        acc.zero();
-        int j = a + sp;
-        // four independent gathers in flight per lane, then their products
-        for (; j + 3 * split < b; j += 4 * split) {
-            const Vec<Ln::W> x0 = Vec<Ln::W>::load(xb + (size_t)s_col[j] * K);
-            const Vec<Ln::W> x1 = Vec<Ln::W>::load(xb + (size_t)s_col[j + split] * K);
-            const Vec<Ln::W> x2 = Vec<Ln::W>::load(xb + (size_t)s_col[j + 2 * split] * K);
-            const Vec<Ln::W> x3 = Vec<Ln::W>::load(xb + (size_t)s_col[j + 3 * split] * K);
-            acc.fma(x0, s_val[j]);
-            acc.fma(x1, s_val[j + split]);
-            acc.fma(x2, s_val[j + 2 * split]);
-            acc.fma(x3, s_val[j + 3 * split]);
+    for (int rb = r0; rb < r1; rb += slots) {
+        const int r = rb + slot;
+        const bool on = r < r1;
+        const int a = on ? m.row_ptr[r] - n0 : 0, b = on ? m.row_ptr[r + 1] - n0 : 0;
+        // a row much longer than the item's others is left to the whole wave
+        // below: its lanes alone would walk it in a chain of gathers while
+        // the others wait (power-law rows, 2^11 .. 2^18 of them: 1.3 to 1.9
+        // times as fast; with every row above 16 entries per lane taken so,
+        // uniform rows ran half as fast)
+        const bool wide = b - a > kSpmmWide * split && (b - a) * nrows > 2 * n;
+        unsigned long long todo = __ballot(wide && lane % lpr == 0);
+        if (on && !wide) {
+            Vec<Ln::W> acc;
+            acc.zero();
+            int j = a + sp;
+            // four independent gathers in flight per lane, then their products
+            for (; j + 3 * split < b; j += 4 * split) {
+                const Vec<Ln::W> x0 = Vec<Ln::W>::load(xb + (size_t)s_col[j] * K);
+                const Vec<Ln::W> x1 = Vec<Ln::W>::load(xb + (size_t)s_col[j + split] * K);
+                const Vec<Ln::W> x2 = Vec<Ln::W>::load(xb + (size_t)s_col[j + 2 * split] * K);
+                const Vec<Ln::W> x3 = Vec<Ln::W>::load(xb + (size_t)s_col[j + 3 * split] * K);
+                acc.fma(x0, s_val[j]);
+                acc.fma(x1, s_val[j + split]);
+                acc.fma(x2, s_val[j + 2 * split]);
+                acc.fma(x3, s_val[j + 3 * split]);
+            }
+            for (; j < b; j += split) acc.fma_from(xb + (size_t)s_col[j] * K, s_val[j]);
+            // the lanes of one row run the same iterations, so the shuffles
+            // below only read lanes that are active
+            for (int msk = Ln::V; msk < lpr; msk <<= 1) acc.shfl_add(msk);
+            if (sp == 0) acc.add_to(m.y + (size_t)r * K + v * Ln::W);
         }
-        for (; j < b; j += split) acc.fma_from(xb + (size_t)s_col[j] * K, s_val[j]);
-        // the lanes of one row run the same iterations, so the shuffles below
-        // only read lanes that are active
-        for (int msk = Ln::V; msk < lpr; msk <<= 1) acc.shfl_add(msk);
-        if (sp == 0) acc.add_to(m.y + (size_t)r * K + v * Ln::W);
+        while (todo) {
+            const int l = __ffsll((long long)todo) - 1;
+            todo &= todo - 1;
+            const int wa = __builtin_amdgcn_readlane(a, l), wb = __builtin_amdgcn_readlane(b, l);
+            const int wr = __builtin_amdgcn_readlane(r, l);
+            Vec<Ln::W> acc;
+            acc.zero();
+            int j = wa + lane / Ln::V;
+            for (; j + 3 * Ln::SLOTS < wb; j += 4 * Ln::SLOTS) {
+                const Vec<Ln::W> x0 = Vec<Ln::W>::load(xb + (size_t)s_col[j] * K);
+                const Vec<Ln::W> x1 = Vec<Ln::W>::load(xb + (size_t)s_col[j + Ln::SLOTS] * K);
+                const Vec<Ln::W> x2 = Vec<Ln::W>::load(xb + (size_t)s_col[j + 2 * Ln::SLOTS] * K);
+                const Vec<Ln::W> x3 = Vec<Ln::W>::load(xb + (size_t)s_col[j + 3 * Ln::SLOTS] * K);
+                acc.fma(x0, s_val[j]);
+                acc.fma(x1, s_val[j + Ln::SLOTS]);
+                acc.fma(x2, s_val[j + 2 * Ln::SLOTS]);
+                acc.fma(x3, s_val[j + 3 * Ln::SLOTS]);
+            }
+            for (; j < wb; j += Ln::SLOTS) acc.fma_from(xb + (size_t)s_col[j] * K, s_val[j]);
+#pragma unroll
+            for (int msk = Ln::V; msk < 64; msk <<= 1) acc.shfl_add(msk);
+            if (lane < Ln::V) acc.add_to(m.y + (size_t)wr * K + v * Ln::W);
+        }
     }
     wave_lds_sync();  // the next item reuses this wave's LDS
 }
@@ -203,11 +245,12 @@ __device__ void spmm_block(const SpmmMat& m, int b0, int b1, int lane) {
     (void)G;
 }
 
-__global__ __launch_bounds__(256) void spmm_kernel(const SpmmMat* __restrict__ mats, const int4* __restrict__ items,
+__global__ __launch_bounds__(256, 8) void spmm_kernel(const SpmmMat* __restrict__ mats, const int4* __restrict__ items,
                                                    int n_items, float* __restrict__ carry) {
     __shared__ int s_col[4][kSpmmStageNnz];
     __shared__ float s_val[4][kSpmmStageNnz];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);  // wave-uniform: scalar descriptors
     const int waves = gridDim.x * 4;
     for (int it = blockIdx.x * 4 + w; it < n_items; it += waves) {
         const int4 d = items[it];
@@ -239,21 +282,32 @@ __global__ __launch_bounds__(256) void spmm_kernel(const SpmmMat* __restrict__ m
     }
 }
 
-// One thread per (long row, right-hand side): y += carries in chunk order,
-// summed in FP64 (the cross-workgroup part of a long row's sum).
+// One wave per long row: lane 16 q + j adds carries q, q + 4, ... of
+// right-hand side j in FP64 (the cross-workgroup part of a long row's sum),
+// eight loads in flight, then the four classes are added.
 __global__ __launch_bounds__(256) void spmm_finalize_kernel(const SpmmMat* __restrict__ mats,
                                                             const int4* __restrict__ longs, int n_long,
                                                             const float* __restrict__ carry) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    const int i = t >> 4, j = t & 15;
+    const int i = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
     if (i >= n_long) return;
+    const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
     const int4 d = longs[i];  // {mat, row, first slot, chunks}
     const SpmmMat m = mats[d.x];
-    if (j >= m.k) return;
-    double s = 0.0;
-    for (int c = 0; c < d.w; ++c) s += (double)carry[(size_t)(d.z + c) * 16 + j];
+    const bool out = q == 0 && j < m.k;
     float* yp = m.y + (size_t)d.y * m.k + j;
-    *yp = (float)((double)*yp + s);
+    const float yo = out ? *yp : 0.f;
+    const float* cp = carry + (size_t)d.z * 16 + lane;  // chunk q, right-hand side j
+    double s = 0.0;
+    for (int c = q; c < d.w; c += 32) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = c + 4 * u < d.w && j < m.k ? cp[(size_t)(c - q + 4 * u) * 16] : 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) s += (double)v[u];
+    }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (out) *yp = (float)((double)yo + s);
 }
 
 }  // namespace dev
@@ -265,7 +319,7 @@ int launch_spmm(const DevSpmm& b, hipStream_t st) {
         if (e) return e;
     }
     if (b.n_long > 0) {
-        hipLaunchKernelGGL(dev::spmm_finalize_kernel, dim3((b.n_long * 16 + 255) / 256), dim3(256), 0, st, b.mats,
+        hipLaunchKernelGGL(dev::spmm_finalize_kernel, dim3((b.n_long + 3) / 4), dim3(256), 0, st, b.mats,
                            b.longs, b.n_long, b.carry);
         return (int)hipGetLastError();
     }

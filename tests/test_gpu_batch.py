@@ -138,3 +138,24 @@ def test_batch_bsr_refuses_k1_and_bad_blocks(ctx):
         with pytest.raises(L.ClspmvError):
             B.Batch(ctx, [mat], [k])
     assert b"batch" in L.lib().clspmv_last_error()
+
+
+@pytest.mark.parametrize("k", [1, 4, 16])
+def test_batch_rows_wider_than_their_item(ctx, k):
+    # STREAM items that mix short rows with rows left to the whole wave:
+    # lengths around 24 entries per lane and twice the item's mean, first,
+    # last and next to each other, and long rows of 1 .. 40 carry chunks
+    rng = np.random.default_rng(31)
+    lens = [24, 1, 25, 1, 1, 200, 256, 2, 0, 25] * 9 + [256] + [1] * 63 + [255, 3] * 3 + [257, 1024, 1025, 9000, 40000]
+    rows = np.repeat(np.arange(len(lens)), lens).astype(np.int32)
+    cols = np.concatenate([np.sort(rng.choice(50000, n, replace=False)) for n in lens]).astype(np.int32)
+    vals = rng.standard_normal(rows.size).astype(np.float32)
+    coo = M.CooMatrix.from_arrays(rows, cols, vals, 50000, len(lens))
+    b = B.Batch(ctx, [M.coo2csr(coo)], [k])
+    x = rng.uniform(-1, 1, (coo.width, k)).astype(np.float32)
+    y0 = rng.uniform(-1, 1, (coo.height, k)).astype(np.float32)
+    b.set_x(0, x)
+    b.set_y(0, y0)
+    b.run(1)
+    _check_all(b, [coo], [x], [y0], f"wide rows k={k}")
+    b.free()
