@@ -8,10 +8,11 @@
 //    of a wave reads 1 KiB of contiguous HBM.  x is read as float4 at the
 //    block's float4 column (guarded at the right matrix edge).
 //  * BCSR: the reference gives every block row a 128-thread workgroup with an
-//    LDS tree reduction (A/kernels/spmv_bcsr.cl:4-44).  Here a group of L
-//    lanes (L from the mean blocks per block row) strides the blocks of one
-//    block row and reduces with shuffles, so short block rows do not idle a
-//    whole workgroup.
+//    LDS tree reduction (A/kernels/spmv_bcsr.cl:4-44).  Here block rows are
+//    regrouped at upload (bcsr_group_kernel: one to eight lanes per block
+//    row, 64 lanes' blocks side by side, rows of similar length in a wave);
+//    a part with a few block rows far longer than the rest keeps the arrays
+//    as they are, L lanes striding a block row (bcsr_kernel).
 //  * BSR r x c: element-major values data[e*stride + i]; same L-lane scheme.
 #include "kcommon.hpp"
 #include "launch.hpp"
@@ -129,6 +130,94 @@ __global__ __launch_bounds__(256) void bcsr_kernel(const int* __restrict__ rp, c
             const int row = r * BH + h;
             if (row < rows) y[row] += acc[h];
         }
+    }
+}
+
+// Regrouped BCSR: a workgroup owns 256 / L block rows, the longest first
+// (lane[]: blocks << 16 | row - row0), L lanes per row; block L p + t of a
+// row is lane t's at step p, and a step stores 64 columns and, per float4 of
+// the block, 64 float4 side by side.  G steps' columns, values and x are in
+// flight at once.  Steps past a row's end hold zeros and multiply 0, not x.
+// EDGE: some block reaches past the last column (x guarded there).
+// Bound by HBM (250,000 block rows of nine 4 x 4 blocks 48 -> 25 us, 6.4
+// TB/s), smaller parts by the chain column -> x of a step (100,003 block
+// rows 22.2 -> 14.0), against 8 lanes striding each row's blocks as bcsr_kernel
+// does: of nine blocks its second round used one lane, and one step's loads
+// were in flight.  Three steps at once measured 1-5 % ahead of four and five;
+// plain loads 15 % ahead of nontemporal ones.
+template <int BH, int W4, int L, bool EDGE>
+__global__ __launch_bounds__(256) void bcsr_group_kernel(const int* __restrict__ row0s, const int* __restrict__ step,
+                                                         const unsigned* __restrict__ lanes,
+                                                         const int* __restrict__ col, const float4* __restrict__ data,
+                                                         const float* __restrict__ x, float* __restrict__ y, int rows,
+                                                         int cols) {
+    constexpr int B = BH * W4, G = B <= 2 ? 4 : B <= 4 ? 3 : B <= 8 ? 2 : 1;
+    const int g = xcd_tile(blockIdx.x, gridDim.x);
+    const int lane = threadIdx.x & 63, t = threadIdx.x % L;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int p0 = step[g * 4 + wave], p1 = step[g * 4 + wave + 1];
+    const unsigned meta = lanes[g * (256 / L) + threadIdx.x / L];
+    const int r = row0s[g] + (int)(meta & 0xffffu);
+    int left = (int)(meta >> 16) - t;  // blocks of the row from this lane's first on
+    const bool out = t == 0 && left > 0;
+    float acc[BH], other[BH], yo[BH];  // rounds of G steps add to the two sums in turn
+#pragma unroll
+    for (int h = 0; h < BH; ++h) {
+        acc[h] = other[h] = 0.f;
+        yo[h] = out && r * BH + h < rows ? y[r * BH + h] : 0.f;
+    }
+    for (int p = p0; p < p1; p += G) {
+        int c4[G];
+        float4 v[G][B], xv[G][W4];
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+            if (p + u < p1) c4[u] = col[(size_t)(p + u) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+            if (p + u < p1)
+#pragma unroll
+                for (int e = 0; e < B; ++e) v[u][e] = data[((size_t)(p + u) * B + e) * 64 + lane];
+#pragma unroll
+        for (int u = 0; u < G; ++u)
+            if (p + u < p1)
+#pragma unroll
+                for (int w4 = 0; w4 < W4; ++w4)
+                    xv[u][w4] = EDGE ? x4load(x, c4[u] + w4, cols) : reinterpret_cast<const float4*>(x)[c4[u] + w4];
+        // each block's products summed by themselves, then the steps' blocks
+        // in pairs: fewer roundings of the row's whole sum than one chain
+        float d[G][BH];
+#pragma unroll
+        for (int u = 0; u < G; ++u) {
+#pragma unroll
+            for (int h = 0; h < BH; ++h) d[u][h] = 0.f;
+            if (p + u < p1) {
+                const bool on = left > 0;
+                left -= L;
+#pragma unroll
+                for (int w4 = 0; w4 < W4; ++w4) {
+                    const float4 q = on ? xv[u][w4] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                    for (int h = 0; h < BH; ++h) d[u][h] = dot4(v[u][w4 * BH + h], q, d[u][h]);
+                }
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < BH; ++h) {
+            float s = d[0][h];
+            if constexpr (G == 2) s += d[1][h];
+            if constexpr (G == 3) s = (s + d[1][h]) + d[2][h];
+            if constexpr (G == 4) s = (s + d[1][h]) + (d[2][h] + d[3][h]);
+            const float next = other[h] + s;
+            other[h] = acc[h];
+            acc[h] = next;
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < BH; ++h) acc[h] = group_sum<L>(acc[h] + other[h]);
+    if (out) {
+#pragma unroll
+        for (int h = 0; h < BH; ++h)
+            if (r * BH + h < rows) y[r * BH + h] = yo[h] + acc[h];
     }
 }
 
@@ -352,8 +441,34 @@ static void launch_bcsr_l(const DevBcsr& m, const float* x, float* y, hipStream_
     }
 }
 
+template <int BH, int W4>
+static void launch_bcsr_groups(const DevBcsr& m, const float* x, float* y, hipStream_t st) {
+    const float4* d4 = reinterpret_cast<const float4*>(m.data);
+#define CLSPMV_BCSR_GROUPS(L, E)                                                                                    \
+    hipLaunchKernelGGL((dev::bcsr_group_kernel<BH, W4, L, E>), dim3(m.ngroups), dim3(256), 0, st, m.row_ptr, m.step, \
+                       m.lane, m.col, d4, x, y, m.rows, m.cols)
+    switch (m.lanes + (m.edge ? 16 : 0)) {
+        case 1: CLSPMV_BCSR_GROUPS(1, false); break;
+        case 2: CLSPMV_BCSR_GROUPS(2, false); break;
+        case 4: CLSPMV_BCSR_GROUPS(4, false); break;
+        case 8: CLSPMV_BCSR_GROUPS(8, false); break;
+        case 17: CLSPMV_BCSR_GROUPS(1, true); break;
+        case 18: CLSPMV_BCSR_GROUPS(2, true); break;
+        case 20: CLSPMV_BCSR_GROUPS(4, true); break;
+        default: CLSPMV_BCSR_GROUPS(8, true); break;
+    }
+#undef CLSPMV_BCSR_GROUPS
+}
+
 int launch_bcsr(const DevBcsr& m, const float* x, float* y, hipStream_t st) {
     if (m.brows == 0) return 0;
+    if (m.step) {
+        if (m.ngroups == 0) return 0;
+#define L_BCSR(BH, W4) launch_bcsr_groups<BH, W4>(m, x, y, st)
+        BH_W4_SWITCH(m.bh, m.w4n, L_BCSR)
+#undef L_BCSR
+        return (int)hipGetLastError();
+    }
 #define L_BCSR(BH, W4) launch_bcsr_l<BH, W4>(m, x, y, st)
     BH_W4_SWITCH(m.bh, m.w4n, L_BCSR)
 #undef L_BCSR

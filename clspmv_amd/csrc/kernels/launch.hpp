@@ -135,10 +135,14 @@ struct DevSbell {
     int S, brows, bh, w4n, rows, cols;
 };
 struct DevBcsr {  // b4csr
-    const int* row_ptr;
+    const int* row_ptr;       // regrouped: first block row of every group
     const int* col;
     const float* data;
     int N4, brows, bh, w4n, rows, cols, lanes;
+    // regrouped (k_block.hip: bcsr_group_kernel), else step is null
+    const int* step;          // first step of every wave (4 per group, + 1)
+    const unsigned* lane;     // per block row: blocks << 16 | row - row0
+    int ngroups, edge;
 };
 struct DevBsr {
     const int* row_ptr;   // lanes > 0: block-CSR row pointer; lanes == 0: slice pointer

@@ -1724,6 +1724,96 @@ int clspmv_part_sbell(clspmv_ctx_t ctx, const clspmv_sbell_matrix* m, int method
     });
 }
 
+// Regrouped BCSR unless a few block rows are so long that one lane group each
+// would be the launch's tail.
+static bool bcsr_regroups(const int* rp, int brows) {
+    int longest = 0;
+    for (int r = 0; r < brows; ++r) longest = std::max(longest, rp[r + 1] - rp[r]);
+    const double mean = brows ? (double)rp[brows] / brows : 0.0;
+    return longest <= 0xffff && longest <= 64 + 4 * mean;
+}
+
+// Lanes per block row: doubled while the rows alone give fewer than
+// kBcsrFillWaves wavefronts and a row still feeds its lanes two blocks each
+// (2048, 4096 and 8192: 14.0, 15.2 and 15.2 us at 100,003 rows of nine
+// blocks, 9.6, 10.5 and 10.4 at 40,000 of sixteen).
+static constexpr long long kBcsrFillWaves = 2048;
+
+static int build_bcsr_groups(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_b4csr_matrix* m) {
+    const int bh = (int)m->b4csr_bheight, w4n = (int)m->b4csr_bwidth / 4, B = bh * w4n;
+    const int rows = m->matinfo.height, cols = m->matinfo.width, brows = m->b4csr_row_num;
+    const int N4 = m->b4csr_aligned_size / 4;
+    const int* rp = m->b4csr_row_ptr;
+    const long long nb = rp[brows];
+    int lanes = 1;
+    while (lanes < 8 && (long long)brows * lanes < 64 * kBcsrFillWaves && nb >= 4LL * lanes * brows) lanes *= 2;
+    const int cap = 256 / lanes, wave_rows = 64 / lanes;
+    const int ng = (brows + cap - 1) / cap;
+    std::vector<int> row0((size_t)std::max(1, ng)), step((size_t)ng * 4 + 1, 0);
+    std::vector<unsigned> lane((size_t)std::max(1, ng) * cap, 0u);
+    bool edge = false;
+#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) reduction(|| : edge) if (ng > 16)
+    for (int g = 0; g < ng; ++g) {
+        const int a = g * cap, b = std::min(brows, a + cap);
+        row0[(size_t)g] = a;
+        unsigned* slot = &lane[(size_t)g * cap];
+        for (int r = a; r < b; ++r) slot[r - a] = (unsigned)(rp[r + 1] - rp[r]) << 16 | (unsigned)(r - a);
+        std::stable_sort(slot, slot + (b - a), [](unsigned u, unsigned v) { return u >> 16 > v >> 16; });
+        for (int w = 0; w < 4; ++w)
+            step[(size_t)g * 4 + w + 1] = ((int)(slot[w * wave_rows] >> 16) + lanes - 1) / lanes;
+        for (int k = rp[a]; k < rp[b]; ++k) edge = edge || 4 * ((long long)m->b4csr_col_id[k] + w4n) > cols;
+    }
+    long long steps = 0;
+    for (size_t i = 1; i < step.size(); ++i) {
+        steps += step[i];
+        if (steps * 64 > INT32_MAX) return CLSPMV_E_TOO_LARGE;
+        step[i] = (int)steps;
+    }
+    std::unique_ptr<int[]> col(new (std::nothrow) int[std::max<size_t>(1, (size_t)steps * 64)]);
+    std::unique_ptr<float[]> data(new (std::nothrow) float[std::max<size_t>(1, (size_t)steps * 64 * B * 4)]);
+    if (!col || !data) return CLSPMV_E_NOMEM;
+#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) if (ng > 16)
+    for (int g = 0; g < ng; ++g) {
+        const size_t s0 = (size_t)step[(size_t)g * 4], s1 = (size_t)step[(size_t)g * 4 + 4];
+        std::memset(col.get() + s0 * 64, 0, (s1 - s0) * 256);  // padding: block column 0
+        std::memset(data.get() + s0 * 64 * B * 4, 0, (s1 - s0) * 1024 * B);
+        for (int i = 0; i < cap; ++i) {
+            const unsigned meta = lane[(size_t)g * cap + i];
+            const int len = (int)(meta >> 16), k0 = len ? rp[row0[(size_t)g] + (int)(meta & 0xffffu)] : 0;
+            const size_t p0 = (size_t)step[(size_t)g * 4 + i / wave_rows];
+            for (int j = 0; j < len; ++j) {
+                const size_t st = p0 + j / lanes;
+                const int q = (i % wave_rows) * lanes + j % lanes;
+                col[st * 64 + q] = m->b4csr_col_id[k0 + j];
+                for (int e = 0; e < B; ++e)
+                    std::memcpy(&data[((st * B + e) * 64 + q) * 4], m->b4csr_data + ((size_t)e * N4 + k0 + j) * 4, 16);
+            }
+        }
+    }
+    DevBcsr d{};
+    int rc = 0;
+    auto up = [&](const void* h, size_t bytes) -> const void* { return rc ? nullptr : p->add(ctx, h, bytes, &rc); };
+    d.row_ptr = (const int*)up(row0.data(), (size_t)ng * 4);
+    d.step = (const int*)up(step.data(), step.size() * 4);
+    d.lane = (const unsigned*)up(lane.data(), (size_t)ng * cap * 4);
+    d.col = (const int*)up(col.get(), (size_t)steps * 256);
+    d.data = (const float*)up(data.get(), (size_t)steps * 1024 * B);
+    if (rc) return rc;
+    d.brows = brows;
+    d.bh = bh;
+    d.w4n = w4n;
+    d.rows = rows;
+    d.cols = cols;
+    d.lanes = lanes;
+    d.ngroups = ng;
+    d.edge = edge;
+    p->bcsr = d;
+    char name[32];
+    std::snprintf(name, sizeof(name), "bcsr%u%u_G%d", m->b4csr_bheight, m->b4csr_bwidth, lanes);
+    fill_info(p, CLSPMV_FMT_BCSR, 0, rows, cols, m->matinfo.nnz, name, 1);
+    return CLSPMV_OK;
+}
+
 int clspmv_part_bcsr(clspmv_ctx_t ctx, const clspmv_b4csr_matrix* m, int method, clspmv_part_t* out) {
     return make_part(ctx, out, [&](clspmv_part_t p) {
         const unsigned bw = m->b4csr_bwidth, bh = m->b4csr_bheight;
@@ -1739,6 +1829,7 @@ int clspmv_part_bcsr(clspmv_ctx_t ctx, const clspmv_b4csr_matrix* m, int method,
             set_error("BCSR block column out of range");
             return CLSPMV_E_INVALID;
         }
+        if (bcsr_regroups(m->b4csr_row_ptr, brows)) return build_bcsr_groups(ctx, p, m);
         int rc = 0;
         p->bcsr.row_ptr = (const int*)p->add(ctx, m->b4csr_row_ptr, ((size_t)brows + 1) * 4, &rc);
         if (rc) return rc;
@@ -1748,7 +1839,8 @@ int clspmv_part_bcsr(clspmv_ctx_t ctx, const clspmv_b4csr_matrix* m, int method,
         if (rc) return rc;
         double mean = brows ? (double)nb / brows : 0.0;
         int lanes = std::min(16, std::max(2, pow2_floor((int)(mean + 0.5))));
-        p->bcsr = DevBcsr{p->bcsr.row_ptr, p->bcsr.col, p->bcsr.data, N / 4, brows, (int)bh, (int)bw / 4, rows, cols, lanes};
+        p->bcsr = DevBcsr{p->bcsr.row_ptr, p->bcsr.col, p->bcsr.data, N / 4, brows, (int)bh, (int)bw / 4, rows, cols,
+                          lanes, nullptr, nullptr, 0, 0};
         char name[32];
         std::snprintf(name, sizeof(name), "bcsr%u%u_L%d", bh, bw, lanes);
         fill_info(p, CLSPMV_FMT_BCSR, 0, rows, cols, m->matinfo.nnz, name, 1);
