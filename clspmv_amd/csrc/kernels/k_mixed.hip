@@ -135,7 +135,7 @@ __device__ __forceinline__ void dia_decode(const unsigned (&w)[W], float s, floa
 // a banded matrix -- it takes the branch-free interior loop, chosen once per
 // workgroup.  With R = 4 a wave's 256 rows are one FP8 slice (a scalar
 // scale load per diagonal).
-template <int CODEC>
+template <int CODEC, bool TRI>
 __global__ __launch_bounds__(256) void dia_mixed_kernel(const int* __restrict__ offsets, const void* __restrict__ data,
                                                         const float* __restrict__ scale, int L, int ndiag, int nsl,
                                                         int offmin, int offmax, const float* __restrict__ x,
@@ -180,35 +180,75 @@ __global__ __launch_bounds__(256) void dia_mixed_kernel(const int* __restrict__ 
     float a[R];
 #pragma unroll
     for (int j = 0; j < R; ++j) a[j] = 0.f;
-    // U diagonals' loads in flight per step, the last step's missing ones
-    // skipped by a wave-uniform test (no serial remainder loop); the sums
-    // keep diagonal order.  Boundary workgroups take the same steps with
-    // bounds-tested x loads: a one-diagonal-at-a-time loop there made those
-    // few workgroups the kernel's tail.
-    constexpr int U = R >= 4 ? 6 : 8;
-    for (int d = 0; d < ndiag; d += U) {
-        unsigned w[U][W];
-        float xv[U][R];
+    if constexpr (TRI) {
+        // S triples of consecutive diagonals in flight per step: the three
+        // diagonals' x runs of a lane are R + 2 consecutive values, loaded
+        // once (8 + 16 bytes instead of three times 16) and used from
+        // registers; the sums keep diagonal order, so the bits are those of
+        // the loop below.
+        constexpr int S = 3;
+        for (int d = 0; d < ndiag; d += 3 * S) {
+            unsigned w[S][3][W];
+            float xv[S][R + 2];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (d + u < ndiag) {
-                word(d + u, w[u]);
-                const int c = row + offsets[d + u];
-                if (interior) {
-                    load_x_run<R>(x, c, xv[u]);
-                } else {
+            for (int s = 0; s < S; ++s)
+                if (d + 3 * s < ndiag) {
 #pragma unroll
-                    for (int j = 0; j < R; ++j) xv[u][j] = xload_m(x, c + j, cols);
+                    for (int u = 0; u < 3; ++u) word(d + 3 * s + u, w[s][u]);
+                    const int c = row + offsets[d + 3 * s];
+                    if (interior) {
+                        float t[R];
+                        load_x_run<R>(x, c + 2, t);
+                        xv[s][0] = x[c], xv[s][1] = x[c + 1];
+#pragma unroll
+                        for (int j = 0; j < R; ++j) xv[s][2 + j] = t[j];
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < R + 2; ++j) xv[s][j] = xload_m(x, c + j, cols);
+                    }
                 }
-            }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (d + u < ndiag) {
-                float v[R];
-                dia_decode<CODEC, R, W>(w[u], slice_scale(d + u), v);
+            for (int s = 0; s < S; ++s)
+                if (d + 3 * s < ndiag)
 #pragma unroll
-                for (int j = 0; j < R; ++j) a[j] = fmaf(v[j], xv[u][j], a[j]);
-            }
+                    for (int u = 0; u < 3; ++u) {
+                        float v[R];
+                        dia_decode<CODEC, R, W>(w[s][u], slice_scale(d + 3 * s + u), v);
+#pragma unroll
+                        for (int j = 0; j < R; ++j) a[j] = fmaf(v[j], xv[s][u + j], a[j]);
+                    }
+        }
+    } else {
+        // U diagonals' loads in flight per step, the last step's missing ones
+        // skipped by a wave-uniform test (no serial remainder loop); the sums
+        // keep diagonal order.  Boundary workgroups take the same steps with
+        // bounds-tested x loads: a one-diagonal-at-a-time loop there made those
+        // few workgroups the kernel's tail.
+        constexpr int U = R >= 4 ? 6 : 8;
+        for (int d = 0; d < ndiag; d += U) {
+            unsigned w[U][W];
+            float xv[U][R];
+    #pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (d + u < ndiag) {
+                    word(d + u, w[u]);
+                    const int c = row + offsets[d + u];
+                    if (interior) {
+                        load_x_run<R>(x, c, xv[u]);
+                    } else {
+    #pragma unroll
+                        for (int j = 0; j < R; ++j) xv[u][j] = xload_m(x, c + j, cols);
+                    }
+                }
+    #pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (d + u < ndiag) {
+                    float v[R];
+                    dia_decode<CODEC, R, W>(w[u], slice_scale(d + u), v);
+    #pragma unroll
+                    for (int j = 0; j < R; ++j) a[j] = fmaf(v[j], xv[u][j], a[j]);
+                }
+        }
     }
     float rs[R];
     if (codec_row_scaled(CODEC)) load_vec<R>(scale + row, rs);  // the scale array has L >= row + R entries
@@ -362,17 +402,23 @@ __global__ __launch_bounds__(XW ? kBsrWinRows : 256) void bsr_mixed_kernel(
 
 int launch_dia_mixed(const DevDiaMixed& m, const float* x, float* y, hipStream_t st) {
     if (m.rows == 0) return 0;
-#define CLSPMV_DIA_MIXED(C)                                                                                     \
-    hipLaunchKernelGGL(dev::dia_mixed_kernel<C>, dim3((m.rows + 256 * dev::dia_rows_per_lane<C>() - 1) /      \
-                                                      (256 * dev::dia_rows_per_lane<C>())),                   \
+#define CLSPMV_DIA_MIXED(C, T)                                                                                  \
+    hipLaunchKernelGGL((dev::dia_mixed_kernel<C, T>), dim3((m.rows + 256 * dev::dia_rows_per_lane<C>() - 1) / \
+                                                           (256 * dev::dia_rows_per_lane<C>())),              \
                        dim3(256), 0, st, m.offsets, m.data, m.scale, m.L, m.ndiag, m.nsl, m.offmin, m.offmax, x, \
                        y, m.rows, m.cols)
+// one row per lane (BF16 hi+lo) reads x coalesced and is bound by its 4-byte
+// values (44 us at 128^3, floor 43): no triples there
+#define CLSPMV_DIA_MIXED_T(C)                 \
+    if (m.triples) CLSPMV_DIA_MIXED(C, true); \
+    else CLSPMV_DIA_MIXED(C, false)
     switch (m.codec) {
-        case kCodecBf16x2: CLSPMV_DIA_MIXED(kCodecBf16x2); break;
-        case kCodecFp16Row: CLSPMV_DIA_MIXED(kCodecFp16Row); break;
-        case kCodecI16Row: CLSPMV_DIA_MIXED(kCodecI16Row); break;
-        default: CLSPMV_DIA_MIXED(kCodecFp8Slice); break;
+        case kCodecBf16x2: CLSPMV_DIA_MIXED(kCodecBf16x2, false); break;
+        case kCodecFp16Row: CLSPMV_DIA_MIXED_T(kCodecFp16Row); break;
+        case kCodecI16Row: CLSPMV_DIA_MIXED_T(kCodecI16Row); break;
+        default: CLSPMV_DIA_MIXED_T(kCodecFp8Slice); break;
     }
+#undef CLSPMV_DIA_MIXED_T
 #undef CLSPMV_DIA_MIXED
     return (int)hipGetLastError();
 }

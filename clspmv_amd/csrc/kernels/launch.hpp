@@ -224,6 +224,7 @@ struct DevDiaMixed {
     const float* scale;   // FP16: L row scales; FP8: ndiag * nsl scales of 256-row slices
     int L, ndiag, nsl, rows, cols, codec;
     int offmin, offmax;   // smallest and largest diagonal offset
+    bool triples;         // the diagonals come in threes of consecutive offsets
 };
 struct DevBsrMixed {
     const int* sp;        // slice pointer of the sliced layout

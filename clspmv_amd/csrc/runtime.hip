@@ -2015,6 +2015,11 @@ int clspmv_part_dia_mixed(clspmv_ctx_t ctx, const clspmv_dia_matrix* m, int code
         d.codec = codec;
         d.offmin = nd ? *std::min_element(m->dia_offsets, m->dia_offsets + nd) : 0;
         d.offmax = nd ? *std::max_element(m->dia_offsets, m->dia_offsets + nd) : 0;
+        // threes of consecutive diagonals share their x loads (any other
+        // pattern, e.g. the 5- and 7-point stencils, takes them one by one)
+        d.triples = nd > 0 && nd % 3 == 0;
+        for (int i = 0; i < nd && d.triples; i += 3)
+            d.triples = m->dia_offsets[i + 1] == m->dia_offsets[i] + 1 && m->dia_offsets[i + 2] == m->dia_offsets[i] + 2;
         p->diam = d;
         p->mixed = true;
         char name[40];
