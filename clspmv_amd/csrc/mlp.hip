@@ -1,9 +1,9 @@
 // The selector network: forward, softmax cross-entropy, backward and Adam,
 // as hand-written HIP kernels (FP32).  A network whose weights fit one CU's
 // LDS (the selector's 24 -> 128 -> 128 -> 22 does) takes two launches per
-// step: mlp_pass_kernel, one workgroup per 16 samples from x to its share of
-// every gradient, and mlp_update_kernel, which adds the shares and takes the
-// Adam step.  Larger networks run layer by layer: an LDS-tiled GEMM kernel
+// step: mlp_pass_kernel, one workgroup per 16 samples from x to the gradient
+// of every layer's input, and mlp_update_kernel, one wave per 16 x 16 tile of
+// the weight gradients, which takes the Adam step too.  Larger networks run layer by layer: an LDS-tiled GEMM kernel
 // with transpose flags, bias / activation and reduction kernels.  Every sum
 // has a fixed order: training is deterministic for a given seed.
 #include <hip/hip_runtime.h>
@@ -138,8 +138,7 @@ struct MlpShape {
     __host__ __device__ int h1() const { return x() + kPassSamples * lds_stride(inp()); }
     __host__ __device__ int h2() const { return h1() + kPassSamples * lds_stride(hp()); }
     __host__ __device__ int z() const { return h2() + kPassSamples * lds_stride(hp()); }
-    __host__ __device__ int losses() const { return z() + kPassSamples * lds_stride(cp()); }
-    __host__ __device__ int floats() const { return losses() + kPassSamples; }
+    __host__ __device__ int floats() const { return z() + kPassSamples * lds_stride(cp()); }
     bool one_cu() const {
         return hid <= kPassHidden && in <= 16 * kPassEnds && cls <= 16 * kPassEnds && floats() <= kPassLds;
     }
@@ -158,13 +157,6 @@ __device__ __forceinline__ void load_rows(const float* __restrict__ src, int row
                     (__attribute__((address_space(3))) void*)(dst + r * stride + c), 4, 0, 0);
 }
 __device__ __forceinline__ void lds_loads_done() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
-
-// The reverse, for the gradients.
-__device__ __forceinline__ void store_rows(const float* src, int stride, int rows, int cols, float* __restrict__ dst,
-                                           int wave, int lane) {
-    for (int r = wave; r < rows; r += kPassWaves)
-        for (int c = lane; c < cols; c += 64) dst[(size_t)r * cols + c] = src[r * stride + c];
-}
 
 // v_mfma_f32_16x16x4f32: lane l gives A[l % 16][l / 16] and B[l / 16][l % 16]
 // and holds rows 4 (l / 16) .. + 3 of column l % 16 of the result.
@@ -202,59 +194,31 @@ __device__ __forceinline__ f32x4 tile_product(const float* a, int am, int ak, co
     return acc;
 }
 
-// N tiles of a weight gradient side by side, acc[t] += A B_t with K = 16
-// samples: B_t is B's columns 16 t .. + 15.  Tiles past `tiles` read whatever
-// LDS holds there (inside the array) and are never stored: no branch between
-// the loads.
-template <int N>
-__device__ __forceinline__ void tile_outer(const float* a, int ak, const float* b, int bk, int lane, f32x4 (&acc)[N]) {
-    const int i = lane & 15, q = lane >> 4;
-    float av[4], bv[N][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) av[u] = a[i + (4 * u + q) * ak];
-#pragma unroll
-    for (int t = 0; t < N; ++t)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) bv[t][u] = b[16 * t + i + (4 * u + q) * bk];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int t = 0; t < N; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[t][u], acc[t], 0, 0, 0);
-}
+// What the passes of a training step hand to mlp_update_kernel, a row per
+// sample: the hidden activations, the gradients of the two hidden layers'
+// and the logits' inputs, the losses.
+struct MlpActs {
+    float *h1, *h2, *d1, *d2, *dz, *loss_i;
+};
 
-__device__ __forceinline__ float sum16(float v) {
-#pragma unroll
-    for (int m = 1; m < 16; m <<= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
-
-__device__ __forceinline__ float column_sum(const float* a, int stride) {
-    float v[kPassSamples], s = 0.f;
-#pragma unroll
-    for (int m = 0; m < kPassSamples; ++m) v[m] = a[m * stride];
-#pragma unroll
-    for (int m = 0; m < kPassSamples; ++m) s += v[m];
-    return s;
-}
-
-// Forward pass of 16 samples at a time and, TRAIN, loss and backward pass:
-// the workgroup's weights stay in LDS, the activations of a tile too, the
-// weight gradients of its tiles in the matrix cores' accumulators (wave w
-// holds rows 16 w .. of W2's and W3's and columns 16 w .. of W1's).  TRAIN
-// writes the workgroup's sums for every parameter and its loss to
-// part[group][params + 1], else the logits to zout.
-// Bound by what one CU can draw and by the chain of layers: 1920 samples of
-// the 24-128-128-22 network are 120 workgroups of 1060 16x16x4 products each
-// and take 27 us, of it 7 the 90 KB of weights coming in, 3 forward, 1
-// softmax, 5 backward, 5 the 90 KB of gradients going out.  A training step
-// is 35-39 us with the update kernel (7 us) against 1340 layer by layer with
-// 20 launches (column sums by one thread per column 330 us, 16 x 16 tiles
-// on the VALU 30 us each).
+// Forward pass of 16 samples at a time and, TRAIN, loss and the gradients of
+// every layer's input: the workgroup's weights stay in LDS, the activations
+// of a tile too.  TRAIN writes them to `acts`, else the logits to zout.  Each
+// sum runs over its terms in ascending order in one chain of fused
+// multiply-adds, as gemm_kernel's and softmax_ce_kernel's do: the same bits.
+// Bound by what one CU can draw (90 KB of weights per workgroup, 7 us) and by
+// the chain of layers.  20 training steps of the 24-128-128-22 network on
+// 1920 samples take 1.11 ms with the update kernel, 28.3 to 29.0 ms layer by
+// layer with 20 launches a step (column sums by one thread per column 330 us,
+// 16 x 16 tiles on the VALU 30 us each), bitwise the same.  Weight gradients
+// kept per workgroup and added afterwards took 0.83 ms, but round differently,
+// and a hidden unit that then changes sides of zero moves the parameters by
+// 1e-5 within a few Adam steps.
 template <bool TRAIN>
 __global__ __launch_bounds__(kPassThreads) void mlp_pass_kernel(MlpShape s, const float* __restrict__ p,
                                                                 const float* __restrict__ x,
                                                                 const int* __restrict__ label, int n,
-                                                                float* __restrict__ part, float* __restrict__ zout) {
+                                                                MlpActs acts, float* __restrict__ zout) {
     __shared__ __align__(16) float lds[kPassLds];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -279,13 +243,13 @@ __global__ __launch_bounds__(kPassThreads) void mlp_pass_kernel(MlpShape s, cons
 
     const bool hidden = 16 * wave < Hp;  // this wave has a tile of the hidden layers
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 d1[kPassEnds], d2[kPassWaves], d3[kPassEnds];
+    // rows row4 .. + 3 of column 16 wave + col of a tile to a samples x cols array
+    auto keep = [&](float* dst, int cols, int s0, const float (&v)[4]) {
+        if (TRAIN && 16 * wave + col < cols)
 #pragma unroll
-    for (int t = 0; t < kPassEnds; ++t) d1[t] = d3[t] = zero;
-#pragma unroll
-    for (int t = 0; t < kPassWaves; ++t) d2[t] = zero;
-    float db1 = 0.f, db2 = 0.f, db3 = 0.f, loss = 0.f;  // column tid's bias gradients; sample tid / 16's losses
-
+            for (int r = 0; r < 4; ++r)
+                if (s0 + row4 + r < n) dst[(size_t)(s0 + row4 + r) * cols + 16 * wave + col] = v[r];
+    };
     for (int s0 = blockIdx.x * kPassSamples; s0 < n; s0 += gridDim.x * kPassSamples) {
         const int live = min(kPassSamples, n - s0);
         load_rows(x + (size_t)s0 * I, live, I, X, is, wave, lane);
@@ -299,14 +263,24 @@ __global__ __launch_bounds__(kPassThreads) void mlp_pass_kernel(MlpShape s, cons
         // hidden layers: column tile `wave` of H1 and H2
         if (hidden) {
             const f32x4 v = tile_product(X, is, 1, W1 + 16 * wave, hs, 1, Ip, lane, zero);
+            float h[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) H1[(row4 + r) * hs + 16 * wave + col] = fmaxf(v[r] + B1[16 * wave + col], 0.f);
+            for (int r = 0; r < 4; ++r) {
+                h[r] = fmaxf(v[r] + B1[16 * wave + col], 0.f);
+                H1[(row4 + r) * hs + 16 * wave + col] = h[r];
+            }
+            keep(acts.h1, H, s0, h);
         }
         __syncthreads();
         if (hidden) {
             const f32x4 v = tile_product(H1, hs, 1, W2 + 16 * wave, hs, 1, Hp, lane, zero);
+            float h[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) H2[(row4 + r) * hs + 16 * wave + col] = fmaxf(v[r] + B2[16 * wave + col], 0.f);
+            for (int r = 0; r < 4; ++r) {
+                h[r] = fmaxf(v[r] + B2[16 * wave + col], 0.f);
+                H2[(row4 + r) * hs + 16 * wave + col] = h[r];
+            }
+            keep(acts.h2, H, s0, h);
         }
         __syncthreads();
         if (16 * wave < Cp) {
@@ -339,97 +313,44 @@ __global__ __launch_bounds__(kPassThreads) void mlp_pass_kernel(MlpShape s, cons
                 for (int d = 1; d < 16; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
                 float ev[kPassEnds], sum = 0.f;
 #pragma unroll
-                for (int k = 0; k < kPassEnds; ++k) {
-                    ev[k] = 16 * k + j < C ? expf(zv[k] - mx) : 0.f;
-                    sum += ev[k];
-                }
-                sum = sum16(sum);
-                float picked = 0.f;
+                for (int k = 0; k < kPassEnds; ++k) ev[k] = 16 * k + j < C ? expf(zv[k] - mx) : 0.f;
+#pragma unroll
+                for (int k = 0; k < kPassEnds; ++k)
+                    for (int c = 0; c < min(16, C - 16 * k); ++c) sum += __shfl(ev[k], (lane & 48) + c, 64);
 #pragma unroll
                 for (int k = 0; k < kPassEnds; ++k)
                     if (16 * k + j < C) {
                         const bool hit = 16 * k + j == t;
-                        zr[16 * k + j] = on ? (ev[k] / sum - (hit ? 1.f : 0.f)) / (float)n : 0.f;
-                        if (hit) picked = zv[k] - mx;
+                        const float dz = on ? (ev[k] / sum - (hit ? 1.f : 0.f)) / (float)n : 0.f;
+                        zr[16 * k + j] = dz;
+                        if (on) acts.dz[(size_t)(s0 + m) * C + 16 * k + j] = dz;
+                        if (on && hit) acts.loss_i[s0 + m] = -(zv[k] - mx - logf(sum));
                     }
-                picked = sum16(picked);
-                if (on && j == 0) loss -= picked - logf(sum);
             }
             __syncthreads();
-            // dW3 += H2^T dZ;  dH2 = dZ W3^T where H2 > 0, in H2's place
-            f32x4 dh = zero;
+            // dH2 = dZ W3^T where H2 > 0, in H2's place (each lane its own)
             if (hidden) {
-                tile_outer<kPassEnds>(H2 + 16 * wave, hs, Z, cs, lane, d3);
-                dh = tile_product(Z, cs, 1, W3 + 16 * wave * cs, 1, cs, Cp, lane, zero);
-            }
-            if (tid < C)
-                db3 += column_sum(Z + tid, cs);
-            __syncthreads();
-            if (hidden) {
+                const f32x4 v = tile_product(Z, cs, 1, W3 + 16 * wave * cs, 1, cs, Cp, lane, zero);
+                float d[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     float* h = H2 + (row4 + r) * hs + 16 * wave + col;
-                    *h = *h <= 0.f ? 0.f : dh[r];
+                    d[r] = *h <= 0.f ? 0.f : v[r];
+                    *h = d[r];
                 }
+                keep(acts.d2, H, s0, d);
             }
             __syncthreads();
-            // dW2 += H1^T dH2;  dH1 = dH2 W2^T where H1 > 0, in H1's place
+            // dH1 = dH2 W2^T where H1 > 0
             if (hidden) {
-                tile_outer<kPassWaves>(H1 + 16 * wave, hs, H2, hs, lane, d2);
-                dh = tile_product(H2, hs, 1, W2 + 16 * wave * hs, 1, hs, Hp, lane, zero);
-            }
-            if (tid < H)
-                db2 += column_sum(H2 + tid, hs);
-            __syncthreads();
-            if (hidden) {
+                const f32x4 v = tile_product(H2, hs, 1, W2 + 16 * wave * hs, 1, hs, Hp, lane, zero);
+                float d[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float* h = H1 + (row4 + r) * hs + 16 * wave + col;
-                    *h = *h <= 0.f ? 0.f : dh[r];
-                }
+                for (int r = 0; r < 4; ++r) d[r] = H1[(row4 + r) * hs + 16 * wave + col] <= 0.f ? 0.f : v[r];
+                keep(acts.d1, H, s0, d);
             }
-            __syncthreads();
-            // dW1 += X^T dH1
-            if (hidden) {
-                tile_outer<kPassEnds>(H1 + 16 * wave, hs, X, is, lane, d1);
-            }
-            if (tid < H)
-                db1 += column_sum(H1 + tid, hs);
         }
         __syncthreads();  // every wave is done with X, H1 and H2
-    }
-    if constexpr (TRAIN) {
-        float* losses = lds + s.losses();
-        if (tid < 16 * kPassSamples && (tid & 15) == 0) losses[tid >> 4] = loss;
-        float* o = part + (size_t)blockIdx.x * (s.params() + 1);
-        float *o1 = o, *ob1 = o1 + I * H, *o2 = ob1 + H, *ob2 = o2 + H * H, *o3 = ob2 + H, *ob3 = o3 + H * C;
-        // through the weights' LDS, so that the stores are whole rows (the
-        // tiles past a matrix' padding are dropped here)
-        if (hidden) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int own = 16 * wave + row4 + r;
-#pragma unroll
-                for (int t = 0; t < kPassWaves; ++t)
-                    if (16 * t < Hp) W2[own * hs + 16 * t + col] = d2[t][r];
-#pragma unroll
-                for (int t = 0; t < kPassEnds; ++t) {
-                    if (16 * t < Cp) W3[own * cs + 16 * t + col] = d3[t][r];
-                    if (16 * t < Ip) W1[(16 * t + col) * hs + own] = d1[t][r];
-                }
-            }
-        }
-        __syncthreads();
-        store_rows(W1, hs, I, H, o1, wave, lane);
-        store_rows(W2, hs, H, H, o2, wave, lane);
-        store_rows(W3, cs, H, C, o3, wave, lane);
-        if (tid < H) ob1[tid] = db1, ob2[tid] = db2;
-        if (tid < C) ob3[tid] = db3;
-        if (tid == 0) {
-            float l = 0.f;
-            for (int m = 0; m < kPassSamples; ++m) l += losses[m];
-            o[s.params()] = l;
-        }
     }
 }
 
@@ -456,48 +377,72 @@ __global__ void adam_kernel(const float* __restrict__ g, long long n, AdamStep a
     v[i] = q.v;
 }
 
-// Gradient i = the sum of the groups' shares (FP64, group class mod 8, then
-// the classes in order), entry np the mean loss; with `update` the Adam step
-// follows.  64 parameters per workgroup, each wave one class, its loads in
-// flight together.
-__global__ __launch_bounds__(kPassThreads) void mlp_update_kernel(const float* __restrict__ part, int groups, int np,
-                                                                  int n, float* __restrict__ g,
-                                                                  float* __restrict__ loss, int update, AdamStep a,
-                                                                  float* __restrict__ p, float* __restrict__ m,
-                                                                  float* __restrict__ v) {
-    __shared__ double sums[kPassWaves][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    AdamState state{0.f, 0.f, 0.f};
-    if (update && w == 0 && i < np) state = AdamState{p[i], m[i], v[i]};  // loads with the shares
-    double s = 0.0;
-    if (i <= np)
-        for (int k = w; k < groups; k += 16 * kPassWaves) {
-            float t[16];
+// Gradients, mean loss and, with `update`, the Adam step.  A workgroup is one
+// wave with one 16 x 16 tile of a weight gradient, P^T Q over the n samples in
+// ascending order in one chain of matrix-core products (the bits of
+// gemm_kernel's chain of fused multiply-adds); a bias gradient and the loss
+// are such tiles with P = 1.  kUpdRows samples' operands are loaded ahead of
+// those that multiply: the chain (8 cycles per sample) then hides most of the
+// loads (20 steps 1.21 ms; 64 rows 1.31, 192 rows 1.29).
+constexpr int kUpdRows = 128;
+__global__ __launch_bounds__(64) void mlp_update_kernel(MlpShape s, const float* __restrict__ x, MlpActs acts, int n,
+                                                        float* __restrict__ g, float* __restrict__ loss, int update,
+                                                        AdamStep a, float* __restrict__ p, float* __restrict__ m,
+                                                        float* __restrict__ v) {
+    const int lane = threadIdx.x, i = lane & 15, q = lane >> 4;
+    const int I = s.in, H = s.hid, C = s.cls, It = s.inp() / 16, Ht = s.hp() / 16, Ct = s.cp() / 16;
+    // the tile: P (null: ones) and Q with their widths, the tile's position
+    // and the offset of the gradient it belongs to
+    const float *P = nullptr, *Q;
+    int pw = 1, qw, ti = 0, tj, off;
+    const int o1 = 0, ob1 = I * H, o2 = ob1 + H, ob2 = o2 + H * H, o3 = ob2 + H, ob3 = o3 + H * C;
+    int b = blockIdx.x;
+    if (b < Ht * Ht) P = acts.h1, pw = H, Q = acts.d2, qw = H, ti = b / Ht, tj = b % Ht, off = o2;
+    else if ((b -= Ht * Ht) < It * Ht) P = x, pw = I, Q = acts.d1, qw = H, ti = b / Ht, tj = b % Ht, off = o1;
+    else if ((b -= It * Ht) < Ht * Ct) P = acts.h2, pw = H, Q = acts.dz, qw = C, ti = b / Ct, tj = b % Ct, off = o3;
+    else if ((b -= Ht * Ct) < Ht) Q = acts.d1, qw = H, tj = b, off = ob1;
+    else if ((b -= Ht) < Ht) Q = acts.d2, qw = H, tj = b, off = ob2;
+    else if ((b -= Ht) < Ct) Q = acts.dz, qw = C, tj = b, off = ob3;
+    else Q = acts.loss_i, qw = 1, tj = 0, off = -1;
+    const int pc = min(16 * ti + i, pw - 1), qc = min(16 * tj + i, qw - 1);  // columns past the edge: never stored
+    constexpr int U = kUpdRows / 4;
+    float pv[U], qv[U];
+    auto load = [&](int k0, float (&pn)[U], float (&qn)[U]) {
+        const bool whole = k0 + kUpdRows <= n;
 #pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const int q = k + u * kPassWaves;
-                t[u] = q < groups ? part[(size_t)q * (np + 1) + i] : 0.f;
-            }
-#pragma unroll
-            for (int u = 0; u < 16; ++u) s += (double)t[u];
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + 4 * u + q, kc = whole ? k : min(k, n - 1);
+            pn[u] = P ? P[(size_t)kc * pw + pc] : 1.f;
+            qn[u] = Q[(size_t)kc * qw + qc];
+            if (k >= n) pn[u] = qn[u] = 0.f;
         }
-    sums[w][lane] = s;
-    __syncthreads();
-    if (w || i > np) return;
-    s = 0.0;
+    };
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    load(0, pv, qv);
+    for (int k0 = 0; k0 < n; k0 += kUpdRows) {
+        float pn[U], qn[U];
+        if (k0 + kUpdRows < n) load(k0 + kUpdRows, pn, qn);
 #pragma unroll
-    for (int k = 0; k < kPassWaves; ++k) s += sums[k][lane];
-    if (i == np) {
-        *loss = (float)(s / (double)n);
+        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(pv[u], qv[u], acc, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) pv[u] = pn[u], qv[u] = qn[u];
+    }
+    if (off < 0) {
+        if (lane == 0) *loss = acc[0] / (float)n;
         return;
     }
-    g[i] = (float)s;
-    if (!update) return;
-    state = adam(a, (float)s, state);
-    p[i] = state.p;
-    m[i] = state.m;
-    v[i] = state.v;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int row = 16 * ti + 4 * q + r, c = 16 * tj + i;
+        if (row >= pw || c >= qw) continue;
+        const int at = off + row * qw + c;
+        g[at] = acc[r];
+        if (!update) continue;
+        const AdamState w = adam(a, acc[r], AdamState{p[at], m[at], v[at]});
+        p[at] = w.p;
+        m[at] = w.m;
+        v[at] = w.v;
+    }
 }
 
 __global__ void argmax_kernel(const float* __restrict__ Z, int n, int c, int* __restrict__ out) {
@@ -521,14 +466,13 @@ struct clspmv_mlp_s {
     long long t = 0;            // Adam steps taken since creation or the last set_params
     DevBuf x, y, h1, h2, z;     // activations for the current n
     DevBuf d1, d2, dz, loss_i, loss;
-    DevBuf part;                // one-CU networks: the workgroups' gradient shares
     int cap = 0;                // samples the activation buffers hold
     MlpShape shape{};
     bool one_cu = false;        // mlp_pass_kernel / mlp_update_kernel (else layer by layer)
     float *W1 = nullptr, *b1 = nullptr, *W2 = nullptr, *b2 = nullptr, *W3 = nullptr, *b3 = nullptr;
     float *gW1 = nullptr, *gb1 = nullptr, *gW2 = nullptr, *gb2 = nullptr, *gW3 = nullptr, *gb3 = nullptr;
     ~clspmv_mlp_s() {
-        for (DevBuf* b : {&p, &g, &m, &v, &x, &y, &h1, &h2, &z, &d1, &d2, &dz, &loss_i, &loss, &part}) b->release();
+        for (DevBuf* b : {&p, &g, &m, &v, &x, &y, &h1, &h2, &z, &d1, &d2, &dz, &loss_i, &loss}) b->release();
     }
     void slice(float* base, float*& w1, float*& c1, float*& w2, float*& c2, float*& w3, float*& c3) const {
         w1 = base;
@@ -553,25 +497,22 @@ struct clspmv_mlp_s {
                                    (float*)p.ptr, (float*)m.ptr, (float*)v.ptr);
             return;
         }
+        const MlpActs acts{(float*)h1.ptr, (float*)h2.ptr, (float*)d1.ptr, (float*)d2.ptr, (float*)dz.ptr,
+                           (float*)loss_i.ptr};
         hipLaunchKernelGGL(mlp_pass_kernel<true>, dim3(groups(n)), dim3(kPassThreads), 0, st(), shape,
-                           (const float*)p.ptr, (const float*)x.ptr, (const int*)y.ptr, n, (float*)part.ptr,
-                           (float*)nullptr);
-        hipLaunchKernelGGL(mlp_update_kernel, dim3((unsigned)(np / 64 + 1)), dim3(kPassThreads), 0, st(),
-                           (const float*)part.ptr, groups(n), (int)np, n, (float*)g.ptr, (float*)loss.ptr, update, a,
+                           (const float*)p.ptr, (const float*)x.ptr, (const int*)y.ptr, n, acts, (float*)nullptr);
+        const int It = shape.inp() / 16, Ht = shape.hp() / 16, Ct = shape.cp() / 16;
+        hipLaunchKernelGGL(mlp_update_kernel, dim3(Ht * Ht + It * Ht + Ht * Ct + 2 * Ht + Ct + 1), dim3(64), 0, st(),
+                           shape, (const float*)x.ptr, acts, n, (float*)g.ptr, (float*)loss.ptr, update, a,
                            (float*)p.ptr, (float*)m.ptr, (float*)v.ptr);
     }
     int ensure(int n) {
         if (n <= cap) return CLSPMV_OK;
         cap = 0;
-        for (DevBuf* b : {&x, &y, &h1, &h2, &z, &d1, &d2, &dz, &loss_i, &part}) b->release();
+        for (DevBuf* b : {&x, &y, &h1, &h2, &z, &d1, &d2, &dz, &loss_i}) b->release();
         int rc = x.alloc((size_t)n * in * 4);
         if (!rc) rc = y.alloc((size_t)n * 4);
         if (!rc) rc = z.alloc((size_t)n * cls * 4);
-        if (one_cu) {
-            if (!rc) rc = part.alloc((size_t)groups(n) * (size_t)(np + 1) * 4);
-            if (!rc) cap = n;
-            return rc;
-        }
         if (!rc) rc = h1.alloc((size_t)n * hid * 4);
         if (!rc) rc = h2.alloc((size_t)n * hid * 4);
         if (!rc) rc = d1.alloc((size_t)n * hid * 4);
@@ -593,7 +534,7 @@ struct clspmv_mlp_s {
     void forward(int n) {
         if (one_cu) {
             hipLaunchKernelGGL(mlp_pass_kernel<false>, dim3(groups(n)), dim3(kPassThreads), 0, st(), shape,
-                               (const float*)p.ptr, (const float*)x.ptr, (const int*)nullptr, n, (float*)nullptr,
+                               (const float*)p.ptr, (const float*)x.ptr, (const int*)nullptr, n, MlpActs{},
                                (float*)z.ptr);
             return;
         }
