@@ -254,8 +254,14 @@ int clspmv_batch_create_entries(clspmv_ctx_t ctx, int n, const clspmv_batch_entr
     // up to 32 four-wave workgroups per CU, four times what is resident: the
     // later ones start as earlier ones end, which evens out items of unequal
     // cost (24 matrices of 2^10 .. 2^18 rows, k = 1, 4 and 16: 252 us with 8
-    // per CU, 242 with 16, 227 with 32, 224 with one item per wave)
-    b->dev.grid = std::max(1, std::min((b->dev.n_items + 3) / 4, 256 * 32));
+    // per CU, 242 with 16, 227 with 32, 224 with one item per wave).  Above
+    // 2^18 items (some 480 entries each) only what is resident: every wave
+    // then takes enough items to even out, and waves that advance together
+    // share the X they gather (24 matrices of 2^16 .. 2^19 rows, about 2^18
+    // items, 1206 us with 8 and 1197 with 32; 80 of 2^14 .. 2^19 2539 and
+    // 2586; 256 of 2^10 .. 2^20 8.43 and 8.73 ms).
+    const int per_cu = b->dev.n_items > (1 << 18) ? 8 : 32;
+    b->dev.grid = std::max(1, std::min((b->dev.n_items + 3) / 4, 256 * per_cu));
     *out = b;
     return CLSPMV_OK;
 }

@@ -159,3 +159,22 @@ def test_batch_rows_wider_than_their_item(ctx, k):
     b.run(1)
     _check_all(b, [coo], [x], [y0], f"wide rows k={k}")
     b.free()
+
+
+@pytest.mark.parametrize("rows", [8192 * 4, 2 ** 18, 2 ** 18 + 1])
+def test_batch_items_around_the_grid_limits(ctx, rows):
+    # one row per item: items fill the resident grid, the larger one, and
+    # one more than the larger one takes; whole numbers, so equal exactly
+    r = np.repeat(np.arange(rows), 2).astype(np.int32)
+    c = ((r * 7 + np.tile([0, 1], rows)) % rows).astype(np.int32)
+    v = (1 + r % 5).astype(np.float32)
+    order = np.lexsort((c, r))
+    coo = M.CooMatrix.from_arrays(r, c[order], v, rows, rows)
+    b = B.Batch(ctx, [M.coo2csr(coo)], [1], [(1, 512, 512)])
+    x, y0 = (np.arange(rows) % 11).astype(np.float32), (np.arange(rows) % 3).astype(np.float32)
+    b.set_x(0, x.reshape(-1, 1))
+    b.set_y(0, y0.reshape(-1, 1))
+    b.run(1)
+    want = y0 + np.bincount(r, v * x[c], minlength=rows)
+    assert np.array_equal(b.get_y(0)[:, 0], want.astype(np.float32))
+    b.free()
