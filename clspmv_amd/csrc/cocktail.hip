@@ -243,8 +243,8 @@ bool xtile_pays(long long rows, long long cols, long long nnz) {
 //  DIA  0/2 one row per thread -> 0; 1/3 four rows per thread -> 1.
 //  ELL  0 -> one row per lane, 1 -> four rows per lane.
 //  SELL, SBELL, BELL, BCSR: one kernel per layout.
-//  CSR  both reference methods -> adaptive row blocks (1): it needs no
-//       tuned workgroup count and balances any row-length distribution.
+//  CSR  both reference methods -> adaptive row groups and blocks (1): no
+//       workgroup count to tune, any row-length distribution balanced.
 //  COO  segmented reduction.
 //  Wide x: see xtile_pays above.
 // Part `which` (0..8: bdia, dia, sbell, bell, bcsr, sell, ell, csr, coo) of

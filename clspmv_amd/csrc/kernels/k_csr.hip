@@ -5,9 +5,12 @@
 //  * csr_vector<L>: L lanes per row (L = 2..64 picked from the mean row
 //    length), DPP/shuffle group reduction.  The reference's CSR-vector uses
 //    a fixed 32-lane "warp" per row (A/kernels/spmv_csr_vector.cl:4-40).
-//  * csr_adaptive: rows of at most 64 entries in row groups (csr_group
-//    below: one to sixteen lanes per row, the entries of 64 lanes
-//    interleaved at upload), longer rows by host-planned blocks:
+//  * csr_adaptive: rows of at most 64 entries in row groups
+//    (csr_adaptive_kernel: one to sixteen lanes per row, the entries of 64
+//    lanes interleaved at upload), the others by host-planned blocks
+//    (csr_block):
+//      STREAM  rows of a group that the groups' layout would pad too much,
+//              up to 64 of them with at most 512 nnz;
 //      VECTOR  one row of 65..1024 nnz: the wave strides the row and
 //              reduces across its 64 lanes;
 //      LONG    one 1024-nnz chunk of a longer row: the wave's partial is
@@ -16,6 +19,7 @@
 #include "kcommon.hpp"
 #include "launch.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace clspmv {
@@ -60,33 +64,91 @@ __global__ __launch_bounds__(256) void csr_vector_kernel(const int* __restrict__
     if (lane == 0 && e > s) y[row] += acc;
 }
 
-// One block of a long row (VECTOR or LONG, DevCsrAdaptive::blocks), by one
-// wave.
-__device__ __forceinline__ void csr_long_block(const DevCsrAdaptive& m, int b, const float* __restrict__ x,
-                                               float* __restrict__ y, int lane) {
-    const int4 blk = m.blocks[b];
-    const int row = blk.x, tag = blk.y, n0 = blk.z, n1 = blk.w;
-    const int* __restrict__ col = m.col;
-    const float* __restrict__ val = m.val;
-    float acc = 0.f;
-    int k = n0 + lane;
-    for (; k + 192 < n1; k += 256) {
-        int c0 = ld_stream(col + k), c1 = ld_stream(col + k + 64), c2 = ld_stream(col + k + 128),
-            c3 = ld_stream(col + k + 192);
-        float v0 = ld_stream(val + k), v1 = ld_stream(val + k + 64), v2 = ld_stream(val + k + 128),
-              v3 = ld_stream(val + k + 192);
-        acc = fmaf(v0, x[c0], acc);
-        acc = fmaf(v1, x[c1], acc);
-        acc = fmaf(v2, x[c2], acc);
-        acc = fmaf(v3, x[c3], acc);
+// U x 64 products of a STREAM block (n <= 64 U entries) to LDS, every load
+// issued before the first use: past the block's end the last entry is read
+// again, as a branch around each load would wait for it (with that, and sums
+// reading eight products at a time, 3000 rows of 1 with a 64 in every 512 take
+// 3.1 us instead of 4.6, 1M 7.0 instead of 10.4).
+template <int U>
+__device__ __forceinline__ void csr_products(const int* __restrict__ col, const float* __restrict__ val, int n,
+                                             const float* __restrict__ x, float* sh, int lane) {
+    int c[U];
+    float v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int k = min(lane + 64 * u, n - 1);
+        c[u] = ld_stream(col + k);
+        v[u] = ld_stream(val + k);
     }
-    for (; k < n1; k += 64) acc = fmaf(ld_stream(val + k), x[ld_stream(col + k)], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) {
-        if (tag < 0)
-            m.carry[-tag - 1] = (double)acc;
-        else
-            y[row] += acc;
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] *= x[c[u]];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (lane + 64 * u < n) sh[lane + 64 * u] = v[u];
+}
+
+// One block of rows (csr_adaptive's and csr_slice's), by one wave:
+//   {row, -(slot + 1)}  LONG, one chunk of a row: its sum to carry[slot]
+//   {row, row + 1}      VECTOR, one row
+//   {r0, r1}            STREAM, up to 64 rows of together at most
+//                       kCsrStreamMaxNnz entries: the products go to LDS (sh,
+//                       the wave's own), lane j sums row r0 + j from there;
+//                       counts holds the rows' entries, a byte each, and a
+//                       scan over the wave gives their offsets.
+// Entries blk.z .. blk.w - 1 of col / val.
+__device__ __forceinline__ void csr_block(int4 blk, const unsigned char* __restrict__ counts,
+                                          const int* __restrict__ col, const float* __restrict__ val,
+                                          const float* __restrict__ x, float* __restrict__ y,
+                                          double* __restrict__ carry, float* sh, int lane) {
+    const int r0 = blk.x, tag = blk.y, n0 = blk.z, n1 = blk.w;
+    if (tag < 0 || tag - r0 == 1) {
+        float acc = 0.f;
+        int k = n0 + lane;
+        for (; k + 192 < n1; k += 256) {
+            int c0 = ld_stream(col + k), c1 = ld_stream(col + k + 64), c2 = ld_stream(col + k + 128),
+                c3 = ld_stream(col + k + 192);
+            float v0 = ld_stream(val + k), v1 = ld_stream(val + k + 64), v2 = ld_stream(val + k + 128),
+                  v3 = ld_stream(val + k + 192);
+            acc = fmaf(v0, x[c0], acc);
+            acc = fmaf(v1, x[c1], acc);
+            acc = fmaf(v2, x[c2], acc);
+            acc = fmaf(v3, x[c3], acc);
+        }
+        for (; k < n1; k += 64) acc = fmaf(ld_stream(val + k), x[ld_stream(col + k)], acc);
+        acc = wave_sum(acc);
+        if (lane == 0) {
+            if (tag < 0)
+                carry[-tag - 1] = (double)acc;
+            else if (n1 > n0)
+                y[r0] += acc;
+        }
+        return;
+    }
+    const int n = n1 - n0;
+    if (n == 0) return;  // a slice without entries in these rows
+    const int r = r0 + lane;
+    const int cnt = r < tag ? (int)counts[r] : 0;
+    const float yo = cnt > 0 ? y[r] : 0.f;
+    if (n <= 128)
+        csr_products<2>(col + n0, val + n0, n, x, sh, lane);
+    else if (n <= 256)
+        csr_products<4>(col + n0, val + n0, n, x, sh, lane);
+    else
+        csr_products<kCsrStreamPerLane>(col + n0, val + n0, n, x, sh, lane);
+    int k = wave_scan(cnt) - cnt;
+    const int e = k + cnt;
+    wave_lds_sync();
+    if (cnt > 0) {
+        float acc = 0.f;
+        for (; k + 8 <= e; k += 8) {
+            float p[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) p[u] = sh[k + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc += p[u];
+        }
+        for (; k < e; ++k) acc += sh[k];
+        y[r] = yo + acc;
     }
 }
 
@@ -164,18 +226,21 @@ __device__ __forceinline__ float csr_group_sum(CsrPairs<MODE>& cur, const f32x2*
 // level with 1024 and 3 % ahead of 256 (the same matrix and 57 others); 4
 // pairs in flight 2 % ahead of 2 and level with 8.
 template <int L>
-__global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptive m, int nlong_wg,
+__global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptive m, int nblock_wg,
+                                                                   int blocks_per_wg,
                                                                    const float* __restrict__ x,
                                                                    float* __restrict__ y) {
     extern __shared__ float xs[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    if ((int)blockIdx.x < nlong_wg) {
-        const int b = blockIdx.x * kCsrWaves + wave;
-        if (b < m.nblocks) csr_long_block(m, b, x, y, lane);
+    if ((int)blockIdx.x < nblock_wg) {
+        // few blocks: a CU each (blocks_per_wg of the waves take one)
+        const int b = blockIdx.x * blocks_per_wg + wave;
+        if (wave < blocks_per_wg && b < m.nblocks)
+            csr_block(m.blocks[b], m.counts, m.col, m.val, x, y, m.carry, xs + wave * kCsrStreamMaxNnz, lane);
         return;
     }
-    const int g = xcd_tile(blockIdx.x - nlong_wg, m.ngroups);
+    const int g = xcd_tile(blockIdx.x - nblock_wg, m.ngroups);
     const CsrGroup d = m.groups[g];
     const int p0 = m.pair[g * kCsrWaves + wave], pairs = m.pair[g * kCsrWaves + wave + 1] - p0;
     const int t = threadIdx.x % L;
@@ -217,11 +282,9 @@ __global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptiv
     if (out) *yp = yo + acc;
 }
 
-// One column slice of the column-sliced CSR.  Same block kinds as
-// csr_adaptive_kernel; STREAM blocks take each row's entry count from one
-// byte per row (`counts`) and an exclusive wave scan gives the offsets.  All
-// x reads of a launch fall in one slice of columns, small enough to stay in
-// L2 while the entry streams pass through with nontemporal loads.
+// One column slice of the column-sliced CSR, in blocks of rows.  All x reads
+// of a launch fall in one slice of columns, small enough to stay in L2 while
+// the entry streams pass through with nontemporal loads.
 __global__ __launch_bounds__(256) void csr_slice_kernel(const unsigned char* __restrict__ counts,
                                                         const int* __restrict__ col, const float* __restrict__ val,
                                                         const int4* __restrict__ blocks, int nblocks,
@@ -229,57 +292,9 @@ __global__ __launch_bounds__(256) void csr_slice_kernel(const unsigned char* __r
                                                         double* __restrict__ carry) {
     __shared__ float lds[4][kCsrStreamMaxNnz];
     const int wid = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
     const int b = blockIdx.x * 4 + wid;
     if (b >= nblocks) return;
-    const int4 blk = blocks[b];
-    const int r0 = blk.x, tag = blk.y, n0 = blk.z, n1 = blk.w;
-    if (tag < 0 || tag - r0 == 1) {
-        float acc = 0.f;
-        int k = n0 + lane;
-        for (; k + 192 < n1; k += 256) {
-            int c0 = ld_stream(col + k), c1 = ld_stream(col + k + 64), c2 = ld_stream(col + k + 128),
-                c3 = ld_stream(col + k + 192);
-            float v0 = ld_stream(val + k), v1 = ld_stream(val + k + 64), v2 = ld_stream(val + k + 128),
-                  v3 = ld_stream(val + k + 192);
-            acc = fmaf(v0, x[c0], acc);
-            acc = fmaf(v1, x[c1], acc);
-            acc = fmaf(v2, x[c2], acc);
-            acc = fmaf(v3, x[c3], acc);
-        }
-        for (; k < n1; k += 64) acc = fmaf(ld_stream(val + k), x[ld_stream(col + k)], acc);
-        acc = wave_sum(acc);
-        if (lane == 0) {
-            if (tag < 0)
-                carry[-tag - 1] = (double)acc;
-            else if (n1 > n0)
-                y[r0] += acc;
-        }
-        return;
-    }
-    const int n = n1 - n0;
-    float* sh = lds[wid];
-#pragma unroll
-    for (int u = 0; u < kCsrStreamPerLane; ++u) {
-        const int k = lane + 64 * u;
-        if (k < n) sh[k] = ld_stream(val + n0 + k) * x[ld_stream(col + n0 + k)];
-    }
-    const int r = r0 + lane;
-    const int cnt = (r < tag) ? (int)counts[r] : 0;
-    // exclusive scan of the counts across the wave
-    int incl = cnt;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        int up = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += up;
-    }
-    const int off = incl - cnt;
-    wave_lds_sync();
-    if (cnt > 0) {
-        float acc = 0.f;
-        for (int k = off; k < off + cnt; ++k) acc += sh[k];
-        y[r] += acc;
-    }
+    csr_block(blocks[b], counts, col, val, x, y, carry, lds[wid], threadIdx.x & 63);
 }
 
 __global__ __launch_bounds__(256) void csr_long_finalize_kernel(const int* __restrict__ long_rows,
@@ -322,9 +337,10 @@ int launch_csr_vector(const DevCsr& m, int lanes, const float* x, float* y, hipS
 
 template <int L>
 static void csr_adaptive_launch(const DevCsrAdaptive& m, const float* x, float* y, hipStream_t st) {
-    const int nlong_wg = (m.nblocks + kCsrWaves - 1) / kCsrWaves;
-    hipLaunchKernelGGL(dev::csr_adaptive_kernel<L>, dim3(nlong_wg + m.ngroups), dim3(kCsrThreads),
-                       (size_t)m.lds_floats * 4, st, m, nlong_wg, x, y);
+    const int per_wg = std::min(kCsrWaves, std::max(1, m.nblocks / 256));
+    const int nblock_wg = (m.nblocks + per_wg - 1) / per_wg;
+    hipLaunchKernelGGL(dev::csr_adaptive_kernel<L>, dim3(nblock_wg + m.ngroups), dim3(kCsrThreads),
+                       (size_t)m.lds_floats * 4, st, m, nblock_wg, per_wg, x, y);
 }
 
 int launch_csr_adaptive(const DevCsrAdaptive& m, const float* x, float* y, hipStream_t st) {

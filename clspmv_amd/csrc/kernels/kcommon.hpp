@@ -155,6 +155,18 @@ __device__ __forceinline__ float wave_total(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Inclusive scan (sums) over the 64 lanes, every lane active, in the DPP moves
+// of wave_total.
+__device__ __forceinline__ int wave_scan(int v) {
+    v += dpp_i<0x111, 0xf>(v);
+    v += dpp_i<0x112, 0xf>(v);
+    v += dpp_i<0x114, 0xf>(v);
+    v += dpp_i<0x118, 0xf>(v);
+    v += dpp_i<0x142, 0xa>(v);
+    v += dpp_i<0x143, 0xc>(v);
+    return v;
+}
+
 // Orders LDS traffic among the lanes of one wavefront (no workgroup barrier:
 // the waves of a workgroup may be on different code paths).
 __device__ __forceinline__ void wave_lds_sync() {

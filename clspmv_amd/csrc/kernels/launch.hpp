@@ -24,7 +24,8 @@ struct DevCsr {
     int rows;
 };
 // Adaptive CSR (k_csr.hip): rows of 1..kCsrStreamMaxRowLen entries in row
-// groups of one workgroup each, longer rows in blocks of one wave each.
+// groups of one workgroup each, longer rows and the rows of groups that would
+// be mostly padding in blocks of one wave each.
 constexpr int kCsrThreads = 512;
 constexpr int kCsrWaves = kCsrThreads / 64;
 constexpr int kCsrPairs = 4;          // entry pairs per lane in flight
@@ -47,11 +48,12 @@ struct DevCsrAdaptive {
     const float* gval;        // 64 lanes x 2 values per pair
     const void* gcol;         // 64 lanes x 2 columns per pair, 16 or 32 bits each
     int ngroups, lanes;       // lanes per row: 1, 2, 4, 8 or 16
-    int lds_floats;           // the widest staged x range
-    // longer rows: {row, row + 1 or -(slot + 1), n0, n1}, entries n0 .. n1 - 1 of col / val
+    int lds_floats;           // the widest staged x range, or the STREAM blocks' products
+    // blocks {r0, r1 or -(slot + 1), n0, n1}, entries n0 .. n1 - 1 of col / val
     const int* col;
     const float* val;
     const int4* blocks;
+    const unsigned char* counts;  // entries of each row in a STREAM block (null: there is none)
     int nblocks;
     double* carry;            // one partial per long-row chunk
     const int* long_rows;     // row id of every long row

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -749,11 +750,26 @@ int csr_group_lanes(long long rows, long long nnz) {
 // 12.4 unstaged and 10.9 staged; small matrices did not care.
 constexpr long long kCsrStagePays = 2;
 
+// A group whose waves, padded to their longest row, hold more bytes than its
+// rows in CSR runs as STREAM blocks instead: padding is read and multiplied
+// too, and the wave of the longest rows ends last.  1M rows near the diagonal,
+// groups and blocks: lengths 1..16 (0.75 times CSR's bytes) 14.0 and 18.7 us,
+// one row of 64 in 16, the others of 2 (1.15 times) 17.8 and 15.3, power-law
+// lengths of exponent 1.8 (1.4 times) 18.5 and 15.4, one row of 64 in 512 rows
+// of 1 (4.5 times) 17.4 and 7.0.  With columns all over (int32 each) lengths
+// 1..16 (1.0 times) 62.5 and 59.4, 1..64 (1.09 times) 214 and 206, one of 64
+// in 16 (1.5 times) 48.9 and 43.8.  Several lanes per row round each row up to
+// 2 lanes entries, but their matrices are small and wait for one row's chain:
+// half as many bytes again are taken there (3000 rows of 1..64, 1.14 times:
+// 3.2 and 4.0 us; 30,000 with one of 64 in 16, 1.35 times: 3.8 and 3.5).
+constexpr double kCsrPadOne = 1.0, kCsrPadLanes = 1.5;
+
 // Builds the adaptive layout (DevCsrAdaptive) from CSR arrays (any column
 // order within a row).  Row groups take the rows of 1..kCsrStreamMaxRowLen
 // entries in order, kCsrThreads / lanes of them each (fewer where their
 // distance would not fit 16 bits), the longest first within the group;
-// longer rows become VECTOR / LONG blocks over compacted arrays.
+// longer rows become VECTOR / LONG blocks, the rows of groups with too much
+// padding STREAM blocks, over compacted arrays.
 int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const int* ci, const float* cv, int rows) {
     auto len = [&](int r) { return rp[r + 1] - rp[r]; };
     long long short_rows = 0, short_nnz = 0;
@@ -781,9 +797,10 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
         }
         ++n;
     }
-    const int ng = (int)begin.size();
+    int ng = (int)begin.size();
     begin.push_back(rows);
     std::vector<CsrGroup> groups((size_t)ng);
+    std::vector<unsigned char> stream((size_t)ng);  // the group's rows go to STREAM blocks
     std::vector<unsigned> lane((size_t)std::max(1, ng) * cap, 0u);
     std::vector<int> pair((size_t)ng * kCsrWaves + 1, 0);  // pairs of each wave, then their prefix
 #pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) if (ng > 16)
@@ -810,16 +827,43 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
             if (l == 0 || l > kCsrStreamMaxRowLen) continue;
             slot[at[kCsrStreamMaxRowLen - l]++] = (unsigned)l << 16 | (unsigned)(r - row0);
         }
-        for (int w = 0; w < kCsrWaves; ++w)
-            pair[(size_t)g * kCsrWaves + w + 1] = ((int)(slot[w * wave_rows] >> 16) + 2 * lanes - 1) / (2 * lanes);
+        int gr = 0;  // rows of the group
+        while (gr < cap && slot[gr]) ++gr;
+        long long slots = 0;  // entries of its rows with their padding
+        for (int w = 0; w < kCsrWaves; ++w) {
+            const int np = ((int)(slot[w * wave_rows] >> 16) + 2 * lanes - 1) / (2 * lanes);
+            pair[(size_t)g * kCsrWaves + w + 1] = np;
+            slots += 2LL * lanes * np * std::max(0, std::min(wave_rows, gr - w * wave_rows));
+        }
         CsrGroup& d = groups[(size_t)g];
         d.row0 = row0;
         d.x0 = lo & ~3;  // staged in 16-byte loads
         d.xn = hi - d.x0 + 1;
         d.mode = d.xn <= kCsrWindow && d.xn <= kCsrStagePays * gn ? kCsrStaged : d.xn <= 65536 ? kCsrNear : kCsrWide;
+        const bool wide = d.mode == kCsrWide;
+        stream[(size_t)g] = slots * (wide ? 8 : 6) > (8 * gn + 4 * gr) * (lanes > 1 ? kCsrPadLanes : kCsrPadOne);
     }
+    // the rows of such groups become blocks; the others close ranks
+    std::vector<std::pair<int, int>> stream_rows;
+    int kept = 0;
+    for (int g = 0; g < ng; ++g) {
+        if (stream[(size_t)g]) {
+            stream_rows.push_back({begin[(size_t)g], begin[(size_t)g + 1]});
+            continue;
+        }
+        if (kept != g) {
+            groups[(size_t)kept] = groups[(size_t)g];
+            std::copy_n(&lane[(size_t)g * cap], cap, &lane[(size_t)kept * cap]);
+            std::copy_n(&pair[(size_t)g * kCsrWaves + 1], kCsrWaves, &pair[(size_t)kept * kCsrWaves + 1]);
+        }
+        ++kept;
+    }
+    ng = kept;
+    groups.resize((size_t)ng);
+    lane.resize((size_t)std::max(1, ng) * cap);
+    pair.resize((size_t)ng * kCsrWaves + 1);
     long long pairs = 0, col256 = 0;
-    int lds_floats = 0;
+    int lds_floats = stream_rows.empty() ? 0 : kCsrWaves * kCsrStreamMaxNnz;
     for (int g = 0; g < ng; ++g) {
         groups[(size_t)g].pair0 = (int)pairs;
         groups[(size_t)g].col256 = (int)col256;
@@ -858,14 +902,15 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
             }
         }
     }
-    // the long rows' blocks, over their entries only
+    // the blocks, over their rows' entries only
     std::vector<int4> blocks;
-    std::vector<int> long_rows, long_first{0}, long_at;
-    int slots = 0, long_nnz = 0;
+    std::vector<int> long_rows, long_first{0};
+    std::vector<std::array<int, 3>> runs;  // rows [first, second) start at entry `third` of the compacted arrays
+    int slots = 0, block_nnz = 0;
     for (int r : long_list) {
-        const int n0 = long_nnz, n1 = n0 + len(r);
-        long_at.push_back(n0);
-        long_nnz = n1;
+        const int n0 = block_nnz, n1 = n0 + len(r);
+        runs.push_back({r, r + 1, n0});
+        block_nnz = n1;
         if (len(r) <= kCsrLongChunk) {
             blocks.push_back(make_int4(r, r + 1, n0, n1));
             continue;
@@ -877,14 +922,33 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
         }
         long_first.push_back(slots);
     }
-    std::unique_ptr<int[]> lcol(new (std::nothrow) int[(size_t)std::max(1, long_nnz)]);
-    std::unique_ptr<float[]> lval(new (std::nothrow) float[(size_t)std::max(1, long_nnz)]);
+    for (const auto& range : stream_rows)
+        for (int r = range.first; r < range.second;) {
+            if (len(r) > kCsrStreamMaxRowLen) {
+                ++r;
+                continue;
+            }
+            const int r0 = r;
+            int n = 0;
+            for (; r < range.second && r - r0 < 64; ++r) {
+                if (len(r) > kCsrStreamMaxRowLen || n + len(r) > kCsrStreamMaxNnz) break;
+                n += len(r);
+            }
+            if (n == 0) continue;
+            runs.push_back({r0, r, block_nnz});
+            blocks.push_back(make_int4(r0, r, block_nnz, block_nnz + n));
+            block_nnz += n;
+        }
+    std::vector<unsigned char> counts(stream_rows.empty() ? 0 : (size_t)rows);
+    for (int r = 0; r < (int)counts.size(); ++r) counts[(size_t)r] = (unsigned char)std::min(255, len(r));
+    std::unique_ptr<int[]> lcol(new (std::nothrow) int[(size_t)std::max(1, block_nnz)]);
+    std::unique_ptr<float[]> lval(new (std::nothrow) float[(size_t)std::max(1, block_nnz)]);
     if (!lcol || !lval) return CLSPMV_E_NOMEM;
-#pragma omp parallel for schedule(dynamic, 16) num_threads(omp_threads()) if (long_nnz > 65536)
-    for (long long i = 0; i < (long long)long_list.size(); ++i) {
-        const int r = long_list[(size_t)i];
-        std::copy(ci + rp[r], ci + rp[r + 1], lcol.get() + long_at[(size_t)i]);
-        std::copy(cv + rp[r], cv + rp[r + 1], lval.get() + long_at[(size_t)i]);
+#pragma omp parallel for schedule(dynamic, 64) num_threads(omp_threads()) if (block_nnz > 65536)
+    for (long long i = 0; i < (long long)runs.size(); ++i) {
+        const auto& q = runs[(size_t)i];  // consecutive rows: their entries lie together
+        std::copy(ci + rp[q[0]], ci + rp[q[1]], lcol.get() + q[2]);
+        std::copy(cv + rp[q[0]], cv + rp[q[1]], lval.get() + q[2]);
     }
     DevCsrAdaptive d{};
     int rc = 0;
@@ -896,8 +960,9 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
     d.lane = (const unsigned*)up(lane.data(), lane.size() * 4);
     d.gval = (const float*)up(gval.get(), (size_t)pairs * 512);
     d.gcol = up(gcol.get(), (size_t)col256 * 256);
-    d.col = (const int*)up(lcol.get(), (size_t)long_nnz * 4);
-    d.val = (const float*)up(lval.get(), (size_t)long_nnz * 4);
+    d.col = (const int*)up(lcol.get(), (size_t)block_nnz * 4);
+    d.val = (const float*)up(lval.get(), (size_t)block_nnz * 4);
+    if (!counts.empty()) d.counts = (const unsigned char*)up(counts.data(), counts.size());
     d.blocks = (const int4*)up(blocks.data(), blocks.size() * sizeof(int4));
     d.long_rows = (const int*)up(long_rows.data(), long_rows.size() * 4);
     d.long_first = (const int*)up(long_first.data(), long_first.size() * 4);

@@ -1,8 +1,8 @@
 """The adaptive CSR part's row groups (k_csr.hip: csr_adaptive_kernel) at the
 edges of their layout: row lengths around the 64-entry limit, empty rows,
 rows too far apart for 16-bit offsets, x ranges around the staged window and
-the 16-bit columns, every number of lanes per row, and padding next to an
-infinite x entry.  Tolerance: the FP32 bar of oracle.parity_report."""
+the 16-bit columns, every number of lanes per row, padding next to an infinite
+x entry, and skewed row lengths, whose groups become STREAM blocks.  Tolerance: the FP32 bar of oracle.parity_report."""
 import numpy as np
 import pytest
 
@@ -84,3 +84,49 @@ def test_padding_keeps_infinities_out(ctx, span):
     x[0] = np.inf
     y, _ = gpu_spmv(ctx, L.FMT_CSR_VECTOR, M.coo2csr(coo), x, y0, 1)
     assert np.isinf(y[0]) and np.isfinite(y[1:]).all()
+
+
+def _one_in(n, rows, rest, seed=0):
+    lens = np.full(rows, rest)
+    lens[seed % n::n] = 64
+    return lens
+
+
+def _power_law(rows, exponent, seed):
+    return np.minimum(np.random.default_rng(seed).zipf(exponent, rows), 64)
+
+
+def _mixed_groups():
+    # even and skewed groups in turn; empty and long rows within and between
+    # the skewed ones; the last group is partly filled
+    lens = np.concatenate([_lens(512, 5, 9, 1), _one_in(256, 512, 1), _lens(512, 1, 3, 2), _one_in(512, 512, 2, 511),
+                           _one_in(100, 77, 1)])
+    lens[512 + 40:512 + 60] = 0
+    lens[[512 + 3, 512 + 200, 1023, 1600, 2000, lens.size - 1]] = [65, 2000, 1024, 1025, 100, 70]
+    return lens
+
+
+SKEWED = {
+    "one row of 64 in 512": lambda: _one_in(512, 20000, 1),
+    "one row of 64 in 64": lambda: _one_in(64, 20000, 2),
+    "64 first in a group of one": lambda: _one_in(600, 500, 1),
+    "power law 2.5": lambda: _power_law(20011, 2.5, 1),
+    "power law 1.8": lambda: _power_law(20011, 1.8, 2),
+    "even and skewed groups": _mixed_groups,
+}
+
+
+@pytest.mark.parametrize("width", [4000, 200000])
+@pytest.mark.parametrize("name", SKEWED)
+def test_skewed_groups_are_not_padded(ctx, name, width):
+    lens = SKEWED[name]()
+    coo = _rows(lens, width, 31)
+    x, y0 = M.gen_vector(coo.width, 32), M.gen_vector(coo.height, 33)
+    y, info = gpu_spmv(ctx, L.FMT_CSR_VECTOR, M.coo2csr(coo), x, y0, 1)
+    rep = O.parity_report(y, coo, x, y0)
+    assert rep["ok"], (name, info, rep)
+    # at most 1.5 times the entries and row pointers of CSR (several lanes per
+    # row), and beside them 5 bytes per row and 16 per 8 rows or per block, a
+    # group's descriptors and the long rows' lists
+    csr = 8 * coo.nnz + 4 * (lens.size + 1)
+    assert info["stored_bytes"] <= 1.5 * csr + 8 * lens.size + 1024, (name, info, csr)
