@@ -1789,8 +1789,15 @@ int clspmv_part_sbell(clspmv_ctx_t ctx, const clspmv_sbell_matrix* m, int method
     });
 }
 
-// Regrouped BCSR unless a few block rows are so long that one lane group each
-// would be the launch's tail.
+// Block rows are regrouped unless one is so long that its lane group alone
+// would be the launch's tail, or the waves, padded to their longest row, would
+// hold more than this many times the blocks.  250,000 rows of 4 x 4 blocks,
+// regrouped and as they are: 1..16 blocks a row (1.2 times) 28.9 and 36.7 us,
+// 100,000 rows of 1..9 (1.35 times) 10.2 and 10.4, one row of 64 in 64 rows of
+// 3 (4.6 times) 53.4 and 29.8, in 256 rows of 1 (13 times) 44.6 and 31.1.
+// Between lies no clear line (one row of 64 in 16 of 3, 2.7 times: 54.2 and
+// 66.6); the padding is device memory too.
+static constexpr double kBcsrPad = 1.5;
 static bool bcsr_regroups(const int* rp, int brows) {
     int longest = 0;
     for (int r = 0; r < brows; ++r) longest = std::max(longest, rp[r + 1] - rp[r]);
@@ -1804,7 +1811,9 @@ static bool bcsr_regroups(const int* rp, int brows) {
 // blocks, 9.6, 10.5 and 10.4 at 40,000 of sixteen).
 static constexpr long long kBcsrFillWaves = 2048;
 
-static int build_bcsr_groups(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_b4csr_matrix* m) {
+// Regroups the block rows into p; *padded (and p untouched) where that would
+// pad them too much.
+static int build_bcsr_groups(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_b4csr_matrix* m, bool* padded) {
     const int bh = (int)m->b4csr_bheight, w4n = (int)m->b4csr_bwidth / 4, B = bh * w4n;
     const int rows = m->matinfo.height, cols = m->matinfo.width, brows = m->b4csr_row_num;
     const int N4 = m->b4csr_aligned_size / 4;
@@ -1817,23 +1826,25 @@ static int build_bcsr_groups(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_b4c
     std::vector<int> row0((size_t)std::max(1, ng)), step((size_t)ng * 4 + 1, 0);
     std::vector<unsigned> lane((size_t)std::max(1, ng) * cap, 0u);
     bool edge = false;
-#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) reduction(|| : edge) if (ng > 16)
+    long long slots = 0;  // blocks with the padding of their waves
+#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) reduction(|| : edge) reduction(+ : slots) if (ng > 16)
     for (int g = 0; g < ng; ++g) {
         const int a = g * cap, b = std::min(brows, a + cap);
         row0[(size_t)g] = a;
         unsigned* slot = &lane[(size_t)g * cap];
         for (int r = a; r < b; ++r) slot[r - a] = (unsigned)(rp[r + 1] - rp[r]) << 16 | (unsigned)(r - a);
         std::stable_sort(slot, slot + (b - a), [](unsigned u, unsigned v) { return u >> 16 > v >> 16; });
-        for (int w = 0; w < 4; ++w)
-            step[(size_t)g * 4 + w + 1] = ((int)(slot[w * wave_rows] >> 16) + lanes - 1) / lanes;
+        for (int w = 0; w < 4; ++w) {
+            const int n = ((int)(slot[w * wave_rows] >> 16) + lanes - 1) / lanes;
+            step[(size_t)g * 4 + w + 1] = n;
+            slots += (long long)n * lanes * std::max(0, std::min(wave_rows, b - a - w * wave_rows));
+        }
         for (int k = rp[a]; k < rp[b]; ++k) edge = edge || 4 * ((long long)m->b4csr_col_id[k] + w4n) > cols;
     }
-    long long steps = 0;
-    for (size_t i = 1; i < step.size(); ++i) {
-        steps += step[i];
-        if (steps * 64 > INT32_MAX) return CLSPMV_E_TOO_LARGE;
-        step[i] = (int)steps;
-    }
+    *padded = slots > kBcsrPad * nb;
+    if (*padded) return CLSPMV_OK;
+    long long steps = 0;  // fits an int: 64 blocks a step, at most kBcsrPad times all of them
+    for (size_t i = 1; i < step.size(); ++i) step[i] = (int)(steps += step[i]);
     std::unique_ptr<int[]> col(new (std::nothrow) int[std::max<size_t>(1, (size_t)steps * 64)]);
     std::unique_ptr<float[]> data(new (std::nothrow) float[std::max<size_t>(1, (size_t)steps * 64 * B * 4)]);
     if (!col || !data) return CLSPMV_E_NOMEM;
@@ -1894,7 +1905,11 @@ int clspmv_part_bcsr(clspmv_ctx_t ctx, const clspmv_b4csr_matrix* m, int method,
             set_error("BCSR block column out of range");
             return CLSPMV_E_INVALID;
         }
-        if (bcsr_regroups(m->b4csr_row_ptr, brows)) return build_bcsr_groups(ctx, p, m);
+        if (bcsr_regroups(m->b4csr_row_ptr, brows)) {
+            bool padded = false;
+            const int rc = build_bcsr_groups(ctx, p, m, &padded);
+            if (rc || !padded) return rc;
+        }
         int rc = 0;
         p->bcsr.row_ptr = (const int*)p->add(ctx, m->b4csr_row_ptr, ((size_t)brows + 1) * 4, &rc);
         if (rc) return rc;

@@ -1,8 +1,8 @@
 """The regrouped BCSR kernel (k_block.hip: bcsr_group_kernel) at its edges:
 every block shape, one to eight lanes per block row, ragged and empty block
 rows, a width that no block column divides, one group and one row more, and
-the parts that keep the plain kernel (a block row far longer than the rest);
-padding next to an infinite x entry.  Tolerance: the FP32 bar of
+the parts that keep the plain kernel (a block row far longer than the rest, or
+skewed rows that regrouping would pad); padding next to an infinite x entry.  Tolerance: the FP32 bar of
 oracle.parity_report."""
 import numpy as np
 import pytest
@@ -40,6 +40,7 @@ def _check(ctx, coo, bw, bh, kernel):
     rep = O.parity_report(y, coo, x, y0)
     assert rep["ok"], (info, rep)
     assert kernel in info["kernel"], info
+    return info
 
 
 @pytest.mark.parametrize("width", [804, 803])
@@ -57,6 +58,16 @@ def test_lanes_per_block_row(ctx, rows, lo, hi, lanes):
 
 def test_one_long_block_row_keeps_the_plain_kernel(ctx):
     _check(ctx, _coo([3] * 200 + [400] + [2] * 100, 4, 4, 4000, 7), 4, 4, "_L")
+
+
+@pytest.mark.parametrize("every,rest,kernel", [(256, 1, "_L"), (64, 3, "_L"), (16, 3, "_L"), (3, 40, "_G")])
+def test_skewed_block_rows_are_not_padded(ctx, every, rest, kernel):
+    lens = np.full(2000, rest)
+    lens[5::every] = 64
+    info = _check(ctx, _coo(lens, 4, 4, 4000, every), 4, 4, kernel)
+    # 64 bytes of values and 4 of column a block, 1.5 times the blocks at most
+    # but for the last group's; a few bytes a row beside them
+    assert info["stored_bytes"] <= 1.5 * 68 * lens.sum() + 16 * lens.size + 68 * 256 * 64 / 4
 
 
 def test_padding_keeps_infinities_out(ctx):
