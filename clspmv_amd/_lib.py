@@ -220,6 +220,7 @@ _SIGS = [
     ("clspmv_plan_free", C.c_int, [C.c_void_p]),
     ("clspmv_init_plan_kernels", C.c_int, [C.c_void_p, C.c_void_p, _FP, _FP, _P(C.c_void_p)]),
     ("clspmv_power_iterate", C.c_int, [C.c_void_p, C.c_int]),
+    ("clspmv_power_iterate_launches", C.c_int, [C.c_void_p, C.c_int]),
     ("clspmv_evaluate", C.c_int, [C.c_void_p, _FP, _FP, _FP]),
     ("clspmv_evaluate_report", C.c_int, [C.c_void_p, C.c_void_p, _FP, _FP, _FP, C.c_int, C.c_int, C.c_void_p]),
     ("clspmv_cpy_vector_from_cpu", C.c_int, [C.c_void_p, _FP, C.c_int]),

@@ -232,8 +232,8 @@ class GpuCocktail:
 
 def power_iterate(ctx: Context, gpu: GpuCocktail, k: int):
     """The iteration of A/src/eval.cpp:19-72 (`example`): k times
-    {y += A x; x := y}, device-resident (clspmv_power_iterate: captured
-    graphs, no host round trip); returns y."""
+    {y += A x; x := y}, device-resident (clspmv_power_iterate, no host round
+    trip); returns y."""
     check(lib().clspmv_power_iterate(gpu.h, k), "power_iterate")
     return gpu.result_to_cpu()
 

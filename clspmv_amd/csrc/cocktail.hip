@@ -39,9 +39,9 @@ struct clspmv_gpumat_s {
     // every part covers rows of its own (row runs of the plan): parts may
     // then run side by side on the extra streams below
     bool disjoint = false;
-    // iterations per launch of a matrix that is one narrow-band DIA part (0:
-    // other matrices) and the two vectors its launches alternate between
-    int step_limit = 0;
+    // a matrix that is one narrow-band DIA part takes several iterations per
+    // launch, which alternate between these two vectors
+    bool steps = false;
     DevBuf step[2];
     std::vector<hipStream_t> aux;  // created on first concurrent call
     std::vector<hipEvent_t> ev;    // ev[0]: fork; ev[1 + a]: join of aux[a]
@@ -174,11 +174,15 @@ int enqueue_concurrent(clspmv_gpumat_s* g, int passes, hipStream_t st) {
     return e == hipSuccess ? CLSPMV_OK : hip_status(e, "join");
 }
 
-// `iterations` (>= 2) iterations {y += A x; x := y}, several per launch: the
-// first launch reads x and y, the last writes both, those between alternate
-// between the object's two step vectors.
-int enqueue_steps(clspmv_gpumat_s* g, int iterations, hipStream_t st) {
-    const int launches = std::max(2, (iterations + g->step_limit - 1) / g->step_limit);
+// Launches that `iterations` iterations {y += A x; x := y} are dealt to, 0:
+// one product and one copy each.
+int step_launches(const clspmv_gpumat_s* g, int iterations) {
+    return g->steps && !g_use_graph ? clspmv_part_step_launches(g->parts[0], iterations) : 0;
+}
+
+// Those launches (>= 2): the first reads x and y, the last writes both, those
+// between alternate between the object's two step vectors.
+int enqueue_steps(clspmv_gpumat_s* g, int iterations, int launches, hipStream_t st) {
     float *x = (float*)g->x.ptr, *y = (float*)g->y.ptr;
     const float *xi = x, *yi = y;
     for (int i = 0, done = 0; i < launches; ++i) {
@@ -199,7 +203,8 @@ int run_passes(clspmv_gpumat_s* g, int ntimes, bool iterate) {
     hipStream_t st = g->ctx->stream();
     if (!g_use_graph && !iterate && g_streams && g->disjoint && g->parts.size() > 1 && ntimes > 0)
         return enqueue_concurrent(g, ntimes, st);
-    if (!g_use_graph && iterate && g->step_limit > 0 && ntimes > 1) return enqueue_steps(g, ntimes, st);
+    const int launches = iterate ? step_launches(g, ntimes) : 0;
+    if (launches) return enqueue_steps(g, ntimes, launches, st);
     if (!g_use_graph || g->parts.empty()) return enqueue_passes(g, ntimes, iterate, st);
     for (int done = 0; done < ntimes;) {
         const int n = std::min(kGraphPasses, ntimes - done);
@@ -922,9 +927,9 @@ int init_from_plan(clspmv_ctx_t ctx, const clspmv_plan_s* P, const float* vec, c
         if (g->parts.size() == 1 && g->row0[0] == 0 && g->width == g->height) {
             clspmv_part_info inf;
             clspmv_part_get_info(g->parts[0], &inf);
-            if (inf.rows == g->height && inf.cols == g->width) g->step_limit = clspmv_part_step_limit(g->parts[0]);
+            g->steps = inf.rows == g->height && inf.cols == g->width && clspmv_part_step_limit(g->parts[0]) > 0;
         }
-        if (g->step_limit > 0)
+        if (g->steps)
             for (auto& b : g->step)
                 if (!rc) rc = b.alloc((size_t)g->height * 4);
     }
@@ -1026,6 +1031,10 @@ int clspmv_power_iterate(clspmv_gpumat_t g, int iterations) {
         return CLSPMV_E_INVALID;
     }
     return run_passes(g, iterations, true);
+}
+
+int clspmv_power_iterate_launches(clspmv_gpumat_t g, int iterations) {
+    return g && g->width == g->height ? step_launches(g, iterations) : 0;
 }
 
 int clspmv_cpy_vector_from_cpu(clspmv_gpumat_t g, const float* vec, int n) {

@@ -303,7 +303,7 @@ int launch_dia(const DevDia& m, int method, const float* x, float* y, hipStream_
 template <int D>
 static void dia_steps_launch(const DevDia& m, int steps, int from_zero, const float* x, const float* y, float* xout,
                              float* yout, hipStream_t st) {
-    const int w = dia_step_reach(m), R = dia_step_rows(m);
+    const int w = (int)dia_step_reach(m), R = dia_step_rows(m);
     const dim3 grid((m.rows + R - 1) / R), block(kDiaStepThreads);
     const int rows = std::min(m.rows, R + 2 * steps * w);
 #define CLSPMV_DIA_STEPS(U)                                                                                       \

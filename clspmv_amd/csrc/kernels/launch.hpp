@@ -101,14 +101,37 @@ constexpr int kDiaStepDiags = 8;       // diagonals at most (in registers, per r
 constexpr int kDiaStepSlots = 10;      // rows per thread at most: 8 x 10 diagonal registers
 constexpr int kDiaStepFloats = 20480;  // vector range of one of the two LDS buffers: 80 KiB
 constexpr int kDiaStepGroups = 256;    // workgroups: one per CU
-inline int dia_step_reach(const DevDia& m) { return m.offmax > -m.offmin ? m.offmax : -m.offmin; }
+inline long long dia_step_reach(const DevDia& m) {
+    return m.offmax > -(long long)m.offmin ? m.offmax : -(long long)m.offmin;
+}
 inline int dia_step_rows(const DevDia& m) { return (m.rows + kDiaStepGroups - 1) / kDiaStepGroups; }
+// Whether `iterations` iterations dealt to so many launches beat as many
+// products and copies.
+// A product and a copy take 5 us or more (two launches, up to 7.5 where the
+// host starts them slowly); a launch starts in 3 and reads the
+// diagonals of its whole range, so these have to be few per iteration: from
+// one XCD's 4 MiB L2 where the matrix fits there, else from the Infinity
+// Cache.  Measured (us per iteration, one by one and several per launch; range
+// x diagonals / steps): 65,536 rows of 8 diagonals, w = 2000: 5.0 and 4.5
+// (33,000); of 3, w = 4000 5.0 and 5.8 (25,000, one step fits); 300,000 rows
+// of 3, w = 2000 5.6 and 4.7 (14,000); of 5, w = 2000 5.9 and 6.4 (23,000); of
+// 8, w = 2500 6.0 and 11.6 (49,000, one step).  Large matrices, whose range is
+// mostly their own rows: 1M rows of 8, w = 1000 13.0 and 7.1.
+inline bool dia_steps_pay(const DevDia& m, int iterations, int launches) {
+    const long long R = dia_step_rows(m), steps = (iterations + launches - 1) / launches;
+    const long long with_halo = R + 2 * steps * dia_step_reach(m), range = with_halo < m.rows ? with_halo : m.rows;
+    const bool l2 = (long long)m.rows * m.ndiag <= (1 << 20);
+    return launches * range * m.ndiag <= (l2 ? 55000LL * iterations - 43000LL * launches
+                                             : 20000LL * iterations - 8000LL * launches) ||
+           2 * launches * range <= 3 * R * iterations;
+}
 // Steps one launch takes at most (0: none).  Its range, R rows and steps * w
 // to each side, has to fit the row slots and an LDS buffer; and since a
 // launch costs a start and a read of the range's diagonals while a step costs
 // work for the whole range, the cost per step is least near 100 / sqrt(w)
 // steps: measured best at 6 for w = 256 (65,536 rows), 4 for 512 (262,144)
-// and 3 to 4 for 700 (490,000), 12 for 64.
+// and 3 to 4 for 700 (490,000), 12 for 64.  0 also where no number of steps
+// pays.
 inline int dia_step_limit(const DevDia& m) {
     if (m.rows != m.cols || m.rows < 1 || m.ndiag < 1 || m.ndiag > kDiaStepDiags) return 0;
     const long long w = dia_step_reach(m), R = dia_step_rows(m);
@@ -117,7 +140,17 @@ inline int dia_step_limit(const DevDia& m) {
     long long most = 64;
     while (most > 0 && rows < m.rows && rows < R + 2 * most * w) --most;
     while (most > 1 && most * most * w > 10000) --most;
-    return (int)most;
+    for (int s = 1; s <= most; ++s)
+        if (dia_steps_pay(m, s, 1)) return (int)most;
+    return 0;
+}
+// Launches for that many iterations (at least 2: the first reads x and y, the
+// last writes them), 0 where they go one by one.
+inline int dia_step_launches(const DevDia& m, int iterations) {
+    const int limit = iterations > 1 ? dia_step_limit(m) : 0;
+    if (!limit) return 0;
+    const int n = (int)((iterations + (long long)limit - 1) / limit), launches = n < 2 ? 2 : n;
+    return dia_steps_pay(m, iterations, launches) ? launches : 0;
 }
 struct DevBdia {
     const int* bptr;

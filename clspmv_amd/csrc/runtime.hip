@@ -2203,9 +2203,14 @@ int clspmv_part_launch(clspmv_part_t p, const float* x, float* y, hipStream_t st
     }
 }
 
-int clspmv_part_step_limit(clspmv_part_t p) {
-    if (p->mixed || p->info.format != CLSPMV_FMT_DIA || p->info.method > 1) return 0;
-    return dia_step_limit(p->dia);
+static bool dia_one_step(const clspmv_part_s* p) {  // the kernels whose bits dia_steps_kernel has
+    return !p->mixed && p->info.format == CLSPMV_FMT_DIA && p->info.method <= 1;
+}
+
+int clspmv_part_step_limit(clspmv_part_t p) { return dia_one_step(p) ? dia_step_limit(p->dia) : 0; }
+
+int clspmv_part_step_launches(clspmv_part_t p, int iterations) {
+    return dia_one_step(p) ? dia_step_launches(p->dia, iterations) : 0;
 }
 
 int clspmv_part_launch_steps(clspmv_part_t p, int steps, const float* x, const float* y, float* xout, float* yout,

@@ -31,8 +31,10 @@ struct DevBuf {
 
 extern "C" int clspmv_part_launch(clspmv_part_t p, const float* x, float* y, hipStream_t st);
 // DIA parts of narrow-band square matrices: iterations {y += A x; x := y} one
-// launch can take (0: other parts), and such a launch from x, y into xout
-// (may be null) and yout, which x and y must not overlap.
+// launch can take (0: other parts), the launches that so many iterations are
+// dealt to (0: they go one by one), and such a launch from x, y into xout (may
+// be null) and yout, which x and y must not overlap.
 extern "C" int clspmv_part_step_limit(clspmv_part_t p);
+extern "C" int clspmv_part_step_launches(clspmv_part_t p, int iterations);
 extern "C" int clspmv_part_launch_steps(clspmv_part_t p, int steps, const float* x, const float* y, float* xout,
                                         float* yout, hipStream_t st);

@@ -120,10 +120,13 @@ int clspmv_do_spmv(clspmv_gpumat_t gpumat, int ntimes);
  * cpy_vector_from_gpu :1510-1556): `iterations` times { y += A x; x := y },
  * all enqueued on the device with no host round trip (x := y by a copy
  * kernel; a narrow-band matrix that is one DIA part of at most 8 diagonals
- * takes several iterations per launch instead, the same bits; from captured
- * graphs of up to 64 iterations with "cocktail_graph" 1).  Square matrices
+ * takes several iterations per launch instead where that is faster, the same
+ * bits; from captured graphs of up to 64 iterations with "cocktail_graph" 1).  Square matrices
  * only; asynchronous. */
 int clspmv_power_iterate(clspmv_gpumat_t gpumat, int iterations);
+/* The launches clspmv_power_iterate deals that many iterations to when it
+ * takes several per launch; 0: a product and a copy for each. */
+int clspmv_power_iterate_launches(clspmv_gpumat_t gpumat, int iterations);
 /* cpy_vector_from_cpu / _from_gpu, cpy_result_from_cpu / _from_gpu /
  * _to_cpu / _to_gpu (:1458-1588).  *_gpu take device pointers. */
 int clspmv_cpy_vector_from_cpu(clspmv_gpumat_t gpumat, const float* vec, int vec_size);
