@@ -352,8 +352,7 @@ def batched_c4(ctx, args):
       plain     k_i single-vector FP32 SpMVs per matrix, CSR adaptive row
                 blocks (one launch each);
       selector  the same with the format the learned selector picks;
-      batched   one replay of the captured graph (persistent kernel over all
-                matrices);
+      batched   one replay of the captured graph (one kernel over all matrices);
     and, on a seeded eighth of the matrices, the plain FP32 Cocktail path
     (analyzer + k do_spmv per matrix) against a batch of the same
     matrices."""

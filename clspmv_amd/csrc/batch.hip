@@ -251,17 +251,17 @@ int clspmv_batch_create_entries(clspmv_ctx_t ctx, int n, const clspmv_batch_entr
     b->dev.carry = (float*)b->carry.ptr;
     b->dev.n_items = (int)items.size();
     b->dev.n_long = (int)longs.size();
-    // up to 32 four-wave workgroups per CU, four times what is resident: the
-    // later ones start as earlier ones end, which evens out items of unequal
-    // cost (24 matrices of 2^10 .. 2^18 rows, k = 1, 4 and 16: 252 us with 8
-    // per CU, 242 with 16, 227 with 32, 224 with one item per wave).  Above
-    // 2^18 items (some 480 entries each) only what is resident: every wave
-    // then takes enough items to even out, and waves that advance together
-    // share the X they gather (24 matrices of 2^16 .. 2^19 rows, about 2^18
-    // items, 1206 us with 8 and 1197 with 32; 80 of 2^14 .. 2^19 2539 and
-    // 2586; 256 of 2^10 .. 2^20 8.43 and 8.73 ms).
-    const int per_cu = b->dev.n_items > (1 << 18) ? 8 : 32;
-    b->dev.grid = std::max(1, std::min((b->dev.n_items + 3) / 4, 256 * per_cu));
+    // One item per wave: workgroups start in item order as others end, which
+    // evens out items of unequal cost and keeps the waves at work near each
+    // other, so that they share the X they gather.  Persistent waves that took
+    // every W-th item had several matrices in flight at a time (us with 8 and
+    // 32 workgroups per CU, and so): 4 matrices of 2^20 rows x 32 scattered
+    // entries, k = 1: 1348, 1594, 872; 8 of 2^18, k = 4: 783, 783, 463; 256 of
+    // 2^10 .. 2^20, mixed: 8412, 8630, 6095; 24 of 2^10 .. 2^18 241, 218, 215.
+    // 27-point stencils and blocks, whose X is near by itself, lose up to 4 %
+    // to the starts (4 stencils of 2^20 rows, k = 1: 290, 295, 300).  Runs of
+    // 2 to 8 neighbouring items per wave were slower.
+    b->dev.grid = std::max(1, std::min((b->dev.n_items + 3) / 4, kSpmmGridMax));
     *out = b;
     return CLSPMV_OK;
 }

@@ -1,5 +1,5 @@
 // Batched multi-right-hand-side SpMV: Y_i += A_i X_i for many CSR matrices
-// in one persistent launch, each with k_i in {1, 4, 16} right-hand sides.
+// in one launch, each with k_i in {1, 4, 16} right-hand sides.
 //
 // X_i is stored row-major (x[col*k + j]) and Y_i likewise, so the k values a
 // nonzero multiplies are contiguous: one gather of a 64-byte line serves all
@@ -25,9 +25,9 @@
 //     rows of the block row's current block, column c, times x[col + c]
 //     [4q .. 4q+3], so bdim instructions advance every block row of the
 //     item by one block (see spmm_block).
-// Waves take items i, i + W, i + 2W, ... (W = waves in the grid), so the
-// launch is one grid whatever the number of matrices.  No atomics: results
-// are deterministic.
+// A wave takes one item, so the launch is one grid whatever the number of
+// matrices (beyond kSpmmGridMax workgroups, items i, i + W, ... of W waves).
+// No atomics: results are deterministic.
 // Bound by gathering X: from L2 while a matrix's X fits there, else from the
 // Infinity Cache (2^18 rows x 32 scattered entries, k = 16: 4.6 TB/s of X
 // rows).  Item and matrix descriptors are wave-uniform and live in scalar

@@ -275,6 +275,7 @@ struct DevBsrMixed {
 constexpr int kSpmmStageNnz = 512;    // entries of a STREAM item (staged in LDS)
 constexpr int kSpmmLongChunk = 1024;  // entries of a LONG item
 constexpr int kSpmmWide = 24;         // entries per lane from which a STREAM row may be left to the whole wave
+constexpr int kSpmmGridMax = 1 << 23;  // workgroups of 256: the launch limit is 2^32 threads
 struct SpmmMat {
     const int* row_ptr;  // CSR: rows + 1; BSR: block rows + 1
     const int* col;      // CSR: column; BSR: first column of each block

@@ -6,9 +6,8 @@
  * services that apply many small and large matrices per step.  A batch holds
  * n CSR matrices, matrix i with k_i in {1, 4, 16} right-hand sides, on the
  * device; clspmv_batch_run computes Y_i <- A_i X_i + Y_i for every i in one
- * persistent kernel launch (plus one small kernel when some row is longer
- * than the long-row threshold), optionally replayed from a captured
- * hipGraph.  X_i is cols_i x k_i and Y_i is rows_i x k_i, both row-major
+ * kernel launch (plus one small kernel when some row is longer than the
+ * long-row threshold), optionally replayed from a captured hipGraph.  X_i is cols_i x k_i and Y_i is rows_i x k_i, both row-major
  * (x[col * k + j]), in device buffers owned by the batch.
  */
 #ifndef CLSPMV_BATCH_H_

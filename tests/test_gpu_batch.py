@@ -163,8 +163,9 @@ def test_batch_rows_wider_than_their_item(ctx, k):
 
 @pytest.mark.parametrize("rows", [8192 * 4, 2 ** 18, 2 ** 18 + 1])
 def test_batch_items_around_the_grid_limits(ctx, rows):
-    # one row per item: items fill the resident grid, the larger one, and
-    # one more than the larger one takes; whole numbers, so equal exactly
+    # one row per item and one item per wave: what is resident at a time, many
+    # times as many, and a last workgroup of one item; whole numbers, so equal
+    # exactly
     r = np.repeat(np.arange(rows), 2).astype(np.int32)
     c = ((r * 7 + np.tile([0, 1], rows)) % rows).astype(np.int32)
     v = (1 + r % 5).astype(np.float32)
@@ -175,6 +176,7 @@ def test_batch_items_around_the_grid_limits(ctx, rows):
     b.set_x(0, x.reshape(-1, 1))
     b.set_y(0, y0.reshape(-1, 1))
     b.run(1)
+    assert b.stats()["grid"] == (rows + 3) // 4
     want = y0 + np.bincount(r, v * x[c], minlength=rows)
     assert np.array_equal(b.get_y(0)[:, 0], want.astype(np.float32))
     b.free()
