@@ -53,7 +53,7 @@ int check_csr(const clspmv_csr_matrix* m) {
 
 // Items of matrix i: STREAM blocks of consecutive rows within the tile's
 // caps, LONG chunks for rows above the threshold.
-void plan(int i, const clspmv_csr_matrix* m, const clspmv_spmm_tile& t, std::vector<int4>& items,
+void plan(int i, const clspmv_csr_matrix* m, int k, const clspmv_spmm_tile& t, std::vector<int4>& items,
           std::vector<int4>& longs, int& slots) {
     const int* rp = m->csr_row_ptr;
     const int rows = m->matinfo.height;
@@ -76,7 +76,10 @@ void plan(int i, const clspmv_csr_matrix* m, const clspmv_spmm_tile& t, std::vec
             n += l;
             ++r;
         }
-        items.push_back(make_int4(i, r0, r, 0));
+        const int split = spmm_split(k, r - r0);
+        bool wide = false;
+        for (int q = r0; q < r; ++q) wide = wide || spmm_wide(rp[q + 1] - rp[q], split, r - r0, n);
+        items.push_back(make_int4(i, r0, r, wide));
     }
 }
 
@@ -205,7 +208,7 @@ int clspmv_batch_create_entries(clspmv_ctx_t ctx, int n, const clspmv_batch_entr
             rc = hip_status(hipMemcpyAsync(drp, m->csr_row_ptr, (rows + 1) * 4, hipMemcpyHostToDevice, st), "h2d");
             if (!rc && z) rc = hip_status(hipMemcpyAsync(dcol, m->csr_col_id, z * 4, hipMemcpyHostToDevice, st), "h2d");
             if (!rc && z) rc = hip_status(hipMemcpyAsync(dval, m->csr_data, z * 4, hipMemcpyHostToDevice, st), "h2d");
-            plan(i, m, tiles ? tiles[i] : clspmv_spmm_default_tile(k), items, longs, slots);
+            plan(i, m, k, tiles ? tiles[i] : clspmv_spmm_default_tile(k), items, longs, slots);
             b->nnz += (long long)z;
             b->nnz_rhs += (long long)z * k;
             b->alg_bytes += 8LL * (long long)z + 4LL * ((long long)rows + 1) +

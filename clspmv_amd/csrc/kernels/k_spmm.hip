@@ -7,7 +7,7 @@
 // times.
 //
 // Work items (planned on the host, any mix of matrices):
-//   STREAM {mat, r0, r1, 0}: rows [r0, r1) with at most kSpmmStageNnz
+//   STREAM {mat, r0, r1, wide}: rows [r0, r1) with at most kSpmmStageNnz
 //     entries.  The wave copies the entries' columns and values into its LDS
 //     with coalesced loads, then "slots" of lanes each own rows: k/4 lanes
 //     (one for k <= 4) hold a row's float4 (or float) pieces of x[col][:],
@@ -91,7 +91,9 @@ struct Vec<4> {
     }
 };
 
-template <int K>
+// WIDE: some row may be left to the whole wave (else that code is not there:
+// it costs items without such rows up to 5 %).
+template <int K, bool WIDE>
 __device__ void spmm_stream(const SpmmMat& m, int r0, int r1, int* s_col, float* s_val, int lane) {
     using Ln = SpmmLanes<K>;
     const int n0 = m.row_ptr[r0], n = m.row_ptr[r1] - n0;
@@ -101,10 +103,8 @@ __device__ void spmm_stream(const SpmmMat& m, int r0, int r1, int* s_col, float*
     }
     wave_lds_sync();
     // lanes per row: V (one right-hand-side vector) times `split` lanes that
-    // stride the row's entries, as many as the item's rows leave free
-    const int nrows = r1 - r0;
-    int split = 1;
-    while (split * 2 * Ln::V * nrows <= 64) split *= 2;
+    // stride the row's entries
+    const int nrows = r1 - r0, split = spmm_split(K, nrows);
     const int lpr = Ln::V * split, slots = 64 / lpr;
     const int slot = lane / lpr, sp = (lane / Ln::V) % split, v = lane % Ln::V;
     const float* xb = m.x + v * Ln::W;
@@ -117,8 +117,8 @@ __device__ void spmm_stream(const SpmmMat& m, int r0, int r1, int* s_col, float*
         // the others wait (power-law rows, 2^11 .. 2^18 of them: 1.3 to 1.9
         // times as fast; with every row above 16 entries per lane taken so,
         // uniform rows ran half as fast)
-        const bool wide = b - a > kSpmmWide * split && (b - a) * nrows > 2 * n;
-        unsigned long long todo = __ballot(wide && lane % lpr == 0);
+        const bool wide = WIDE && spmm_wide(b - a, split, nrows, n);
+        unsigned long long todo = WIDE ? __ballot(wide && lane % lpr == 0) : 0;
         if (on && !wide) {
             Vec<Ln::W> acc;
             acc.zero();
@@ -140,7 +140,7 @@ __device__ void spmm_stream(const SpmmMat& m, int r0, int r1, int* s_col, float*
             for (int msk = Ln::V; msk < lpr; msk <<= 1) acc.shfl_add(msk);
             if (sp == 0) acc.add_to(m.y + (size_t)r * K + v * Ln::W);
         }
-        while (todo) {
+        while (WIDE && todo) {
             const int l = __ffsll((long long)todo) - 1;
             todo &= todo - 1;
             const int wa = __builtin_amdgcn_readlane(a, l), wb = __builtin_amdgcn_readlane(b, l);
@@ -266,10 +266,13 @@ __global__ __launch_bounds__(256, 8) void spmm_kernel(const SpmmMat* __restrict_
                 default: spmm_block<16, 4>(m, d.y, d.z, lane); break;
             }
         } else if (d.z >= 0) {
-            switch (m.k) {
-                case 1: spmm_stream<1>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
-                case 4: spmm_stream<4>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
-                default: spmm_stream<16>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
+            switch (m.k * 2 + (d.w != 0)) {
+                case 2: spmm_stream<1, false>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
+                case 3: spmm_stream<1, true>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
+                case 8: spmm_stream<4, false>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
+                case 9: spmm_stream<4, true>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
+                case 32: spmm_stream<16, false>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
+                default: spmm_stream<16, true>(m, d.y, d.z, s_col[w], s_val[w], lane); break;
             }
         } else {
             const int slot = -d.z - 1;

@@ -275,6 +275,19 @@ struct DevBsrMixed {
 constexpr int kSpmmStageNnz = 512;    // entries of a STREAM item (staged in LDS)
 constexpr int kSpmmLongChunk = 1024;  // entries of a LONG item
 constexpr int kSpmmWide = 24;         // entries per lane from which a STREAM row may be left to the whole wave
+// Lanes that stride one row of a STREAM item (beside those of its right-hand
+// sides): as many as the item's rows leave free.
+__host__ __device__ inline int spmm_split(int k, int nrows) {
+    const int v = k >= 4 ? k / 4 : 1;
+    int split = 1;
+    while (split * 2 * v * nrows <= 64) split *= 2;
+    return split;
+}
+// A row of len entries so much longer than the others of its item (nrows rows,
+// n entries) that the whole wave takes it.
+__host__ __device__ inline bool spmm_wide(int len, int split, int nrows, int n) {
+    return len > kSpmmWide * split && len * nrows > 2 * n;
+}
 constexpr int kSpmmGridMax = 1 << 23;  // workgroups of 256: the launch limit is 2^32 threads
 struct SpmmMat {
     const int* row_ptr;  // CSR: rows + 1; BSR: block rows + 1
@@ -288,7 +301,7 @@ struct SpmmMat {
 };
 struct DevSpmm {
     const SpmmMat* mats;
-    const int4* items;   // STREAM {mat, r0, r1, 0} / LONG {mat, row, -(slot+1), chunk} /
+    const int4* items;   // STREAM {mat, r0, r1, wide rows} / LONG {mat, row, -(slot+1), chunk} /
                          // BLOCK {mat, block row 0, block row 1, 0} of a BSR matrix
     const int4* longs;   // {mat, row, first carry slot, chunks}
     float* carry;        // 16 floats per LONG item
