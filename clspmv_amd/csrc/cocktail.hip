@@ -43,7 +43,7 @@ struct clspmv_gpumat_s {
     // launch, which alternate between these two vectors
     bool steps = false;
     DevBuf step[2];
-    std::vector<hipStream_t> aux;  // created on first concurrent call
+    std::vector<hipStream_t> aux;
     std::vector<hipEvent_t> ev;    // ev[0]: fork; ev[1 + a]: join of aux[a]
     ~clspmv_gpumat_s() {
         for (auto s : aux) (void)hipStreamSynchronize(s);
@@ -141,9 +141,14 @@ int pass_graph(clspmv_gpumat_s* g, int passes, bool iterate, hipGraphExec_t* out
     return CLSPMV_OK;
 }
 
-// `passes` passes with part j on stream j mod kStreams (see g_streams).
-int enqueue_concurrent(clspmv_gpumat_s* g, int passes, hipStream_t st) {
-    const int ns = (int)std::min<size_t>(kStreams, g->parts.size());
+// Streams that do_spmv runs the parts on, the context's included.
+int num_streams(const clspmv_gpumat_s* g) { return (int)std::min<size_t>(kStreams, g->parts.size()); }
+bool side_by_side(const clspmv_gpumat_s* g) { return !g_use_graph && g_streams && g->disjoint && g->parts.size() > 1; }
+
+// The extra streams and the events that fork and join them (10 to 20 ms: at
+// init, not in the first do_spmv, unless the options changed in between).
+int make_streams(clspmv_gpumat_s* g) {
+    const int ns = num_streams(g);
     while ((int)g->aux.size() < ns - 1) {
         hipStream_t s = nullptr;
         hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
@@ -156,6 +161,13 @@ int enqueue_concurrent(clspmv_gpumat_s* g, int passes, hipStream_t st) {
         if (e != hipSuccess) return hip_status(e, "hipEventCreate");
         g->ev.push_back(ev);
     }
+    return CLSPMV_OK;
+}
+
+// `passes` passes with part j on stream j mod kStreams (see g_streams).
+int enqueue_concurrent(clspmv_gpumat_s* g, int passes, hipStream_t st) {
+    const int rc = make_streams(g), ns = num_streams(g);
+    if (rc) return rc;
     hipError_t e = hipEventRecord(g->ev[0], st);
     for (int a = 0; a < ns - 1 && e == hipSuccess; ++a) e = hipStreamWaitEvent(g->aux[(size_t)a], g->ev[0], 0);
     if (e != hipSuccess) return hip_status(e, "fork");
@@ -201,8 +213,7 @@ int enqueue_steps(clspmv_gpumat_s* g, int iterations, int launches, hipStream_t 
 // then one graph of the remainder.
 int run_passes(clspmv_gpumat_s* g, int ntimes, bool iterate) {
     hipStream_t st = g->ctx->stream();
-    if (!g_use_graph && !iterate && g_streams && g->disjoint && g->parts.size() > 1 && ntimes > 0)
-        return enqueue_concurrent(g, ntimes, st);
+    if (!iterate && ntimes > 0 && side_by_side(g)) return enqueue_concurrent(g, ntimes, st);
     const int launches = iterate ? step_launches(g, ntimes) : 0;
     if (launches) return enqueue_steps(g, ntimes, launches, st);
     if (!g_use_graph || g->parts.empty()) return enqueue_passes(g, ntimes, iterate, st);
@@ -924,6 +935,7 @@ int init_from_plan(clspmv_ctx_t ctx, const clspmv_plan_s* P, const float* vec, c
         g->disjoint = !P->parts.empty();
         for (const PlanPart& q : P->parts) g->disjoint = g->disjoint && q.source == 9;
         // here and not at the first call: that may be under stream capture
+        if (side_by_side(g)) rc = make_streams(g);
         if (g->parts.size() == 1 && g->row0[0] == 0 && g->width == g->height) {
             clspmv_part_info inf;
             clspmv_part_get_info(g->parts[0], &inf);

@@ -3,6 +3,7 @@ do_spmv, compared with the reference's CPU SpMV restated in oracle/ (same
 bound as the single-format tests), on matrices whose partition has one to
 three parts; plus the y = A^k x iteration of A/src/eval.cpp:19-72."""
 import contextlib
+import ctypes as C
 
 import numpy as np
 import pytest
@@ -374,3 +375,39 @@ def test_plan_parity_on_the_selector_family(ctx):
         coo.free()
     # the family reaches the small-matrix layouts
     assert {"dia_lanes", "bsr22_lanes"} & seen, seen
+
+
+def test_first_do_spmv_of_a_plan_under_capture():
+    # what the streams of a plan's row runs need is there before the first
+    # call, which may be under stream capture; each replay is one pass
+    hip = L.lib()  # the HIP runtime's symbols come with the library's
+
+    def call(name, *args):
+        assert getattr(hip, name)(*args) == 0, name
+
+    ctx = M.Context(0)
+    coo = M.gen_cocktail_composite(65536, 77)
+    with _option(b"cocktail_small_plan", 0, 1 << 22):  # runs at this size too
+        plan = CK.Plan.analyze(coo, CK.BenchTables(CK.MI355X_TABLES))
+    assert len(plan.parts()) >= 3 and all(q["source"] == 9 for q in plan.parts())
+    x, y0 = M.gen_vector(coo.width, 1), M.gen_vector(coo.height, 2)
+    a, b = CK.GpuCocktail(ctx, plan, x, y0), CK.GpuCocktail(ctx, plan, x, y0)
+    stream, graph, run = C.c_void_p(), C.c_void_p(), C.c_void_p()
+    call("hipStreamCreate", C.byref(stream))
+    L.check(hip.clspmv_set_stream(ctx.h, stream), "set_stream")
+    call("hipStreamBeginCapture", stream, 1)  # thread-local
+    a.do_spmv(1)
+    call("hipStreamEndCapture", stream, C.byref(graph))
+    call("hipGraphInstantiate", C.byref(run), graph, None, None, C.c_size_t(0))
+    for i in range(3):
+        call("hipGraphLaunch", run, stream)
+        b.do_spmv(1)
+        ya, yb = a.result_to_cpu(), b.result_to_cpu()
+        assert np.array_equal(ya.view(np.uint32), yb.view(np.uint32)), i
+    L.check(hip.clspmv_set_stream(ctx.h, None), "set_stream")
+    call("hipGraphExecDestroy", run)
+    call("hipGraphDestroy", graph)
+    for o in (a, b):
+        o.free()
+    call("hipStreamDestroy", stream)
+    ctx.close()
