@@ -3,9 +3,10 @@
 // LDS (the selector's 24 -> 128 -> 128 -> 22 does) takes two launches per
 // step: mlp_pass_kernel, one workgroup per 16 samples from x to the gradient
 // of every layer's input, and mlp_update_kernel, one wave per 16 x 16 tile of
-// the weight gradients, which takes the Adam step too.  Larger networks run layer by layer: an LDS-tiled GEMM kernel
-// with transpose flags, bias / activation and reduction kernels.  Every sum
-// has a fixed order: training is deterministic for a given seed.
+// the weight gradients, which takes the Adam step too.  Larger networks run
+// layer by layer: an LDS-tiled GEMM kernel with transpose flags, bias /
+// activation and reduction kernels.  Every sum has a fixed order, the same in
+// both: training is deterministic for a given seed.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -83,24 +84,34 @@ __global__ void relu_back_kernel(float* __restrict__ dH, const float* __restrict
     if (i < n && H[i] <= 0.f) dH[i] = 0.f;
 }
 
-// out[j] = sum_i A[i][j] (x scale): one workgroup per 64 columns, its 16
-// waves' row classes (i mod 16) added in order.  (One thread per column took
-// 330 us for 1920 x 128.)
-__global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ A, int M, int N, float scale,
+// out[j] = (sum_i A[i][j], i ascending) / div: one workgroup per 64 columns,
+// whose 16 waves load kColsumRows rows to LDS while the first adds up those
+// before, in order: the chain of mlp_update_kernel's sums, the same bits.
+constexpr int kColsumRows = 128;
+__global__ __launch_bounds__(1024) void colsum_kernel(const float* __restrict__ A, int M, int N, float div,
                                                       float* __restrict__ out) {
-    __shared__ float part[16][64];
+    constexpr int U = kColsumRows / 16;
+    __shared__ float part[2][kColsumRows][64];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int j = blockIdx.x * 64 + lane;
+    const float* col = A + min(j, N - 1);
     float s = 0.f;
-    if (j < N)
-        for (int i = w; i < M; i += 16) s += A[(size_t)i * N + j];
-    part[w][lane] = s;
-    __syncthreads();
-    if (w || j >= N) return;
-    s = 0.f;
+    for (int i0 = 0, b = 0; i0 < M + kColsumRows; i0 += kColsumRows, b ^= 1) {
+        if (i0 < M) {
+            float v[U];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) s += part[k][lane];
-    out[j] = s * scale;
+            for (int u = 0; u < U; ++u) v[u] = col[(size_t)min(i0 + w + 16 * u, M - 1) * N];
+#pragma unroll
+            for (int u = 0; u < U; ++u) part[b][w + 16 * u][lane] = v[u];
+        }
+        if (w == 0 && i0 > 0) {
+            const int n = min(kColsumRows, M - (i0 - kColsumRows));
+#pragma unroll 16
+            for (int i = 0; i < n; ++i) s += part[b ^ 1][i][lane];
+        }
+        __syncthreads();
+    }
+    if (w == 0 && j < N) out[j] = s / div;
 }
 
 // ---------------------------------------------------------------- in one CU
@@ -125,7 +136,6 @@ struct MlpShape {
     __host__ __device__ int inp() const { return pad16(in); }
     __host__ __device__ int hp() const { return pad16(hid); }
     __host__ __device__ int cp() const { return pad16(cls); }
-    __host__ __device__ int params() const { return in * hid + hid + hid * hid + hid + hid * cls + cls; }
     // LDS offsets (floats): the weights and biases, then a tile's x, hidden
     // activations and logits
     __host__ __device__ int w1() const { return 0; }
@@ -205,7 +215,8 @@ struct MlpActs {
 // every layer's input: the workgroup's weights stay in LDS, the activations
 // of a tile too.  TRAIN writes them to `acts`, else the logits to zout.  Each
 // sum runs over its terms in ascending order in one chain of fused
-// multiply-adds, as gemm_kernel's and softmax_ce_kernel's do: the same bits.
+// multiply-adds, as gemm_kernel's, softmax_ce_kernel's and colsum_kernel's do:
+// the same bits.
 // Bound by what one CU can draw (90 KB of weights per workgroup, 7 us) and by
 // the chain of layers.  20 training steps of the 24-128-128-22 network on
 // 1920 samples take 1.11 ms with the update kernel, 28.3 to 29.0 ms layer by
@@ -383,7 +394,7 @@ __global__ void adam_kernel(const float* __restrict__ g, long long n, AdamStep a
 // gemm_kernel's chain of fused multiply-adds); a bias gradient and the loss
 // are such tiles with P = 1.  kUpdRows samples' operands are loaded ahead of
 // those that multiply: the chain (8 cycles per sample) then hides most of the
-// loads (20 steps 1.21 ms; 64 rows 1.31, 192 rows 1.29).
+// loads (64 rows 9 % slower, 192 rows 7 %).
 constexpr int kUpdRows = 128;
 __global__ __launch_bounds__(64) void mlp_update_kernel(MlpShape s, const float* __restrict__ x, MlpActs acts, int n,
                                                         float* __restrict__ g, float* __restrict__ loss, int update,
@@ -526,8 +537,8 @@ struct clspmv_mlp_s {
         hipLaunchKernelGGL(gemm_kernel, dim3((N + kT - 1) / kT, (M + kT - 1) / kT), dim3(kT * kT), 0, st(), M, N,
                            K, A, ta, B, tb, C, acc);
     }
-    void colsum(const float* A, int M, int N, float scale, float* out) {
-        hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((N + 63) / 64)), dim3(1024), 0, st(), A, M, N, scale, out);
+    void colsum(const float* A, int M, int N, float div, float* out) {
+        hipLaunchKernelGGL(colsum_kernel, dim3((unsigned)((N + 63) / 64)), dim3(1024), 0, st(), A, M, N, div, out);
     }
     // Logits of the n uploaded samples (the layers' activations too where
     // the network runs layer by layer).
@@ -553,7 +564,7 @@ struct clspmv_mlp_s {
         float *D1 = (float*)d1.ptr, *D2 = (float*)d2.ptr, *DZ = (float*)dz.ptr;
         hipLaunchKernelGGL(softmax_ce_kernel, blocks(n), dim3(256), 0, st(), Z, (const int*)y.ptr, n, cls, DZ,
                            (float*)loss_i.ptr);
-        colsum((const float*)loss_i.ptr, n, 1, 1.f / (float)n, (float*)loss.ptr);
+        colsum((const float*)loss_i.ptr, n, 1, (float)n, (float*)loss.ptr);
         gemm(hid, cls, n, H2, 1, DZ, 0, gW3, 0);                       // dW3 = H2^T dZ
         colsum(DZ, n, cls, 1.f, gb3);
         gemm(n, hid, cls, DZ, 0, W3, 1, D2, 0);                        // dH2 = dZ W3^T
