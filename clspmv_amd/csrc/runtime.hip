@@ -42,12 +42,14 @@ int DevBuf::upload(clspmv_ctx_t ctx, const void* host, size_t bytes) {
         ptr = nullptr;
         return hip_status(e, "hipMalloc");
     }
-    if (bytes && host) {
-        e = hipMemcpyAsync(ptr, host, bytes, hipMemcpyHostToDevice, ctx->stream());
-        if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream());
-        if (e != hipSuccess) return hip_status(e, "hipMemcpy H2D");
-    }
-    return CLSPMV_OK;
+    return bytes && host ? put(ctx, 0, host, bytes) : CLSPMV_OK;
+}
+
+int DevBuf::put(clspmv_ctx_t ctx, size_t at, const void* host, size_t bytes) {
+    if (!bytes) return CLSPMV_OK;
+    hipError_t e = hipMemcpyAsync(static_cast<char*>(ptr) + at, host, bytes, hipMemcpyHostToDevice, ctx->stream());
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream());
+    return e == hipSuccess ? CLSPMV_OK : hip_status(e, "hipMemcpy H2D");
 }
 
 int DevBuf::alloc(size_t bytes) {
@@ -99,10 +101,11 @@ struct clspmv_part_s {
         *rc = bufs.back().upload(c, host, bytes);
         return bufs.back().ptr;
     }
-    void* scratch(size_t bytes, int* rc) {
+    void* scratch(size_t bytes, int* rc) { return space(bytes, rc).ptr; }
+    DevBuf space(size_t bytes, int* rc) {
         bufs.emplace_back();
         *rc = bufs.back().alloc(bytes);
-        return bufs.back().ptr;
+        return bufs.back();
     }
     ~clspmv_part_s() {
         for (auto& b : bufs) b.release();
@@ -732,6 +735,11 @@ int build_csr_sliced(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const int
     return CLSPMV_OK;
 }
 
+// Layouts made here are uploaded in pieces of at most about this many bytes
+// per array: fresh host arrays of the whole layout cost more in page faults
+// than in copies.
+constexpr size_t kUploadPiece = 8 << 20;
+
 // Lanes per row of the row groups: more of them while the rows alone give
 // fewer than kCsrFillWaves wavefronts (eight per CU) and a row still feeds
 // its lanes a pair each (8000 rows of 20..60 entries: 3.3 us, 8.0 with the
@@ -764,6 +772,25 @@ constexpr long long kCsrStagePays = 2;
 // 3.2 and 4.0 us; 30,000 with one of 64 in 16, 1.35 times: 3.8 and 3.5).
 constexpr double kCsrPadOne = 1.0, kCsrPadLanes = 1.5;
 
+// A row's l entries from its first lane's place on: two to a lane, lane by
+// lane, then on to the wave's next pair.
+template <class Col>
+void csr_lay_row(const float* v, const int* c, int l, int lanes, int x0, float* val, Col* col) {
+    for (int j = 0, t = 0; j < l; j += 2) {
+        val[2 * t] = v[j];
+        col[2 * t] = (Col)(c[j] - x0);
+        if (j + 1 < l) {
+            val[2 * t + 1] = v[j + 1];
+            col[2 * t + 1] = (Col)(c[j + 1] - x0);
+        }
+        if (++t == lanes) {
+            t = 0;
+            val += 128;
+            col += 128;
+        }
+    }
+}
+
 // Builds the adaptive layout (DevCsrAdaptive) from CSR arrays (any column
 // order within a row).  Row groups take the rows of 1..kCsrStreamMaxRowLen
 // entries in order, kCsrThreads / lanes of them each (fewer where their
@@ -773,22 +800,20 @@ constexpr double kCsrPadOne = 1.0, kCsrPadLanes = 1.5;
 int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const int* ci, const float* cv, int rows) {
     auto len = [&](int r) { return rp[r + 1] - rp[r]; };
     long long short_rows = 0, short_nnz = 0;
-    std::vector<int> long_list;  // rows longer than kCsrStreamMaxRowLen
+#pragma omp parallel for schedule(static) num_threads(omp_threads()) reduction(+ : short_rows, short_nnz) if (rows > 65536)
     for (int r = 0; r < rows; ++r) {
         const int l = len(r);
-        if (l > kCsrStreamMaxRowLen) {
-            long_list.push_back(r);
-        } else {
-            short_rows += l > 0;
-            short_nnz += l;
-        }
+        if (l > kCsrStreamMaxRowLen) continue;
+        short_rows += l > 0;
+        short_nnz += l;
     }
     const int lanes = csr_group_lanes(short_rows, short_nnz);
     const int cap = kCsrThreads / lanes, wave_rows = 64 / lanes;
     // rows [begin[g], begin[g + 1]) of group g (rows outside it are skipped)
-    std::vector<int> begin;
+    std::vector<int> begin, long_list;  // long_list: rows longer than kCsrStreamMaxRowLen
     for (int r = 0, n = 0, row0 = 0; r < rows; ++r) {
         const int l = len(r);
+        if (l > kCsrStreamMaxRowLen) long_list.push_back(r);
         if (l == 0 || l > kCsrStreamMaxRowLen) continue;
         if (begin.empty() || n == cap || r - row0 > 0xffff) {
             begin.push_back(r);
@@ -876,31 +901,48 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
         if (groups[(size_t)g].mode == kCsrStaged) lds_floats = std::max(lds_floats, (groups[(size_t)g].xn + 3) & ~3);
         if (col256 > INT32_MAX) return CLSPMV_E_TOO_LARGE;
     }
-    std::unique_ptr<float[]> gval(new (std::nothrow) float[std::max<size_t>(1, (size_t)pairs * 128)]);
-    std::unique_ptr<char[]> gcol(new (std::nothrow) char[std::max<size_t>(1, (size_t)col256 * 256)]);
+    // the groups' entries, laid out and uploaded in pieces of kUploadPiece
+    int rc = 0;
+    DevBuf dval = p->space((size_t)pairs * 512, &rc);
+    if (rc) return rc;
+    DevBuf dcol = p->space((size_t)col256 * 256, &rc);
+    if (rc) return rc;
+    constexpr int piece_pairs = (int)(kUploadPiece / 512), group_pairs = kCsrWaves * kCsrStreamMaxRowLen / 2;
+    const size_t room = (size_t)std::min<long long>(pairs, piece_pairs + group_pairs);
+    std::unique_ptr<float[]> gval(new (std::nothrow) float[std::max<size_t>(1, room * 128)]);
+    std::unique_ptr<char[]> gcol(new (std::nothrow) char[std::max<size_t>(1, room * 512)]);
     if (!gval || !gcol) return CLSPMV_E_NOMEM;
-#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) if (ng > 16)
-    for (int g = 0; g < ng; ++g) {
-        const CsrGroup& d = groups[(size_t)g];
-        const bool wide = d.mode == kCsrWide;
-        const int g0 = d.pair0, g1 = pair[(size_t)(g + 1) * kCsrWaves];
-        char* col = gcol.get() + (size_t)d.col256 * 256;
-        std::memset(gval.get() + (size_t)g0 * 128, 0, (size_t)(g1 - g0) * 512);
-        std::memset(col, 0, (size_t)(g1 - g0) * (wide ? 512 : 256));  // padding: column 0 (wide) or x0
-        for (int i = 0; i < cap; ++i) {
-            const unsigned meta = lane[(size_t)g * cap + i];
-            const int l = (int)(meta >> 16);
-            const int k0 = l ? rp[d.row0 + (int)(meta & 0xffffu)] : 0;
-            const size_t p0 = (size_t)pair[(size_t)g * kCsrWaves + i / wave_rows];
-            for (int j = 0; j < l; ++j) {
-                const size_t q = ((p0 + j / (2 * lanes)) * 64 + (i % wave_rows) * lanes + (j / 2) % lanes) * 2 + j % 2;
-                gval[q] = cv[k0 + j];
+    for (int a = 0, b = 0; a < ng; a = b) {
+        auto first_pair = [&](int g) { return pair[(size_t)g * kCsrWaves]; };
+        for (b = a + 1; b < ng && first_pair(b) - first_pair(a) < piece_pairs;) ++b;
+        const CsrGroup& da = groups[(size_t)a];
+        const long long col_end = b < ng ? groups[(size_t)b].col256 : col256;
+#pragma omp parallel for schedule(static, 4) num_threads(omp_threads()) if (b - a > 16)
+        for (int g = a; g < b; ++g) {
+            const CsrGroup& d = groups[(size_t)g];
+            const bool wide = d.mode == kCsrWide;
+            float* val = gval.get() + (size_t)(d.pair0 - da.pair0) * 128;
+            char* col = gcol.get() + (size_t)(d.col256 - da.col256) * 256;
+            const size_t np = (size_t)(first_pair(g + 1) - d.pair0);
+            std::memset(val, 0, np * 512);
+            std::memset(col, 0, np * (wide ? 512 : 256));  // padding: column 0 (wide) or x0
+            for (int i = 0; i < cap; ++i) {
+                const unsigned meta = lane[(size_t)g * cap + i];
+                const int l = (int)(meta >> 16);
+                if (!l) break;  // the group's last row is behind
+                const int k0 = rp[d.row0 + (int)(meta & 0xffffu)];
+                const size_t p0 = (size_t)(pair[(size_t)g * kCsrWaves + i / wave_rows] - d.pair0);
+                const size_t q = (p0 * 64 + (size_t)(i % wave_rows) * lanes) * 2;
                 if (wide)
-                    reinterpret_cast<int*>(col)[q - (size_t)g0 * 128] = ci[k0 + j];
+                    csr_lay_row(cv + k0, ci + k0, l, lanes, 0, val + q, reinterpret_cast<int*>(col) + q);
                 else
-                    reinterpret_cast<uint16_t*>(col)[q - (size_t)g0 * 128] = (uint16_t)(ci[k0 + j] - d.x0);
+                    csr_lay_row(cv + k0, ci + k0, l, lanes, d.x0, val + q, reinterpret_cast<uint16_t*>(col) + q);
             }
         }
+        rc = dval.put(ctx, (size_t)da.pair0 * 512, gval.get(), (size_t)(first_pair(b) - da.pair0) * 512);
+        if (!rc)
+            rc = dcol.put(ctx, (size_t)da.col256 * 256, gcol.get(), (size_t)(col_end - da.col256) * 256);
+        if (rc) return rc;
     }
     // the blocks, over their rows' entries only
     std::vector<int4> blocks;
@@ -941,27 +983,47 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
         }
     std::vector<unsigned char> counts(stream_rows.empty() ? 0 : (size_t)rows);
     for (int r = 0; r < (int)counts.size(); ++r) counts[(size_t)r] = (unsigned char)std::min(255, len(r));
-    std::unique_ptr<int[]> lcol(new (std::nothrow) int[(size_t)std::max(1, block_nnz)]);
-    std::unique_ptr<float[]> lval(new (std::nothrow) float[(size_t)std::max(1, block_nnz)]);
+    DevBuf dlcol = p->space((size_t)block_nnz * 4, &rc);
+    if (rc) return rc;
+    DevBuf dlval = p->space((size_t)block_nnz * 4, &rc);
+    if (rc) return rc;
+    constexpr int piece_nnz = (int)(kUploadPiece / 4);
+    std::unique_ptr<int[]> lcol(new (std::nothrow) int[(size_t)std::max(1, std::min(block_nnz, piece_nnz))]);
+    std::unique_ptr<float[]> lval(new (std::nothrow) float[(size_t)std::max(1, std::min(block_nnz, piece_nnz))]);
     if (!lcol || !lval) return CLSPMV_E_NOMEM;
-#pragma omp parallel for schedule(dynamic, 64) num_threads(omp_threads()) if (block_nnz > 65536)
-    for (long long i = 0; i < (long long)runs.size(); ++i) {
-        const auto& q = runs[(size_t)i];  // consecutive rows: their entries lie together
-        std::copy(ci + rp[q[0]], ci + rp[q[1]], lcol.get() + q[2]);
-        std::copy(cv + rp[q[0]], cv + rp[q[1]], lval.get() + q[2]);
+    for (size_t a = 0, b = 0; a < runs.size(); a = b) {
+        auto end = [&](size_t i) { return i + 1 < runs.size() ? runs[i + 1][2] : block_nnz; };
+        const int at = runs[a][2];
+        const int *hc = lcol.get();
+        const float* hv = lval.get();
+        if (end(a) - at > piece_nnz) {  // one row: as it lies
+            hc = ci + rp[runs[a][0]];
+            hv = cv + rp[runs[a][0]];
+            b = a + 1;
+        } else {
+            for (b = a + 1; b < runs.size() && end(b) - at <= piece_nnz;) ++b;
+#pragma omp parallel for schedule(dynamic, 64) num_threads(omp_threads()) if (end(b - 1) - at > 65536)
+            for (long long i = (long long)a; i < (long long)b; ++i) {
+                const auto& q = runs[(size_t)i];  // consecutive rows: their entries lie together
+                std::copy(ci + rp[q[0]], ci + rp[q[1]], lcol.get() + (q[2] - at));
+                std::copy(cv + rp[q[0]], cv + rp[q[1]], lval.get() + (q[2] - at));
+            }
+        }
+        rc = dlcol.put(ctx, (size_t)at * 4, hc, (size_t)(end(b - 1) - at) * 4);
+        if (!rc) rc = dlval.put(ctx, (size_t)at * 4, hv, (size_t)(end(b - 1) - at) * 4);
+        if (rc) return rc;
     }
     DevCsrAdaptive d{};
-    int rc = 0;
     auto up = [&](const void* h, size_t bytes) -> const void* {
         return rc ? nullptr : p->add(ctx, h, bytes, &rc);
     };
     d.groups = (const CsrGroup*)up(groups.data(), groups.size() * sizeof(CsrGroup));
     d.pair = (const int*)up(pair.data(), pair.size() * 4);
     d.lane = (const unsigned*)up(lane.data(), lane.size() * 4);
-    d.gval = (const float*)up(gval.get(), (size_t)pairs * 512);
-    d.gcol = up(gcol.get(), (size_t)col256 * 256);
-    d.col = (const int*)up(lcol.get(), (size_t)block_nnz * 4);
-    d.val = (const float*)up(lval.get(), (size_t)block_nnz * 4);
+    d.gval = (const float*)dval.ptr;
+    d.gcol = dcol.ptr;
+    d.col = (const int*)dlcol.ptr;
+    d.val = (const float*)dlval.ptr;
     if (!counts.empty()) d.counts = (const unsigned char*)up(counts.data(), counts.size());
     d.blocks = (const int4*)up(blocks.data(), blocks.size() * sizeof(int4));
     d.long_rows = (const int*)up(long_rows.data(), long_rows.size() * 4);
@@ -1614,24 +1676,12 @@ int clspmv_part_coo(clspmv_ctx_t ctx, const clspmv_coo_matrix* m, int method, cl
             return finish_xtile(p, CLSPMV_FMT_COO, rows, cols, nnz);
         }
         const int chunks = (nnz + kCooChunk - 1) / kCooChunk;
-        const size_t padded = (size_t)chunks * kCooChunk;
-        std::vector<int> rr(padded), cc(padded);
-        std::vector<float> vv(padded, 0.0f);
-        if (nnz) {
-            std::memcpy(rr.data(), m->coo_row_id, (size_t)nnz * 4);
-            std::memcpy(cc.data(), m->coo_col_id, (size_t)nnz * 4);
-            std::memcpy(vv.data(), m->coo_data, (size_t)nnz * 4);
-            for (size_t k = (size_t)nnz; k < padded; ++k) {
-                rr[k] = m->coo_row_id[nnz - 1];
-                cc[k] = m->coo_col_id[nnz - 1];
-            }
-        }
         int rc = 0;
-        p->coo.row = (const int*)p->add(ctx, rr.data(), padded * 4, &rc);
+        p->coo.row = (const int*)p->add(ctx, m->coo_row_id, (size_t)nnz * 4, &rc);
         if (rc) return rc;
-        p->coo.col = (const int*)p->add(ctx, cc.data(), padded * 4, &rc);
+        p->coo.col = (const int*)p->add(ctx, m->coo_col_id, (size_t)nnz * 4, &rc);
         if (rc) return rc;
-        p->coo.val = (const float*)p->add(ctx, vv.data(), padded * 4, &rc);
+        p->coo.val = (const float*)p->add(ctx, m->coo_data, (size_t)nnz * 4, &rc);
         if (rc) return rc;
         p->coo.nnz = nnz;
         p->coo.chunks = chunks;
@@ -1845,35 +1895,58 @@ static int build_bcsr_groups(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_b4c
     if (*padded) return CLSPMV_OK;
     long long steps = 0;  // fits an int: 64 blocks a step, at most kBcsrPad times all of them
     for (size_t i = 1; i < step.size(); ++i) step[i] = (int)(steps += step[i]);
-    std::unique_ptr<int[]> col(new (std::nothrow) int[std::max<size_t>(1, (size_t)steps * 64)]);
-    std::unique_ptr<float[]> data(new (std::nothrow) float[std::max<size_t>(1, (size_t)steps * 64 * B * 4)]);
-    if (!col || !data) return CLSPMV_E_NOMEM;
-#pragma omp parallel for schedule(static, 16) num_threads(omp_threads()) if (ng > 16)
-    for (int g = 0; g < ng; ++g) {
-        const size_t s0 = (size_t)step[(size_t)g * 4], s1 = (size_t)step[(size_t)g * 4 + 4];
-        std::memset(col.get() + s0 * 64, 0, (s1 - s0) * 256);  // padding: block column 0
-        std::memset(data.get() + s0 * 64 * B * 4, 0, (s1 - s0) * 1024 * B);
-        for (int i = 0; i < cap; ++i) {
-            const unsigned meta = lane[(size_t)g * cap + i];
-            const int len = (int)(meta >> 16), k0 = len ? rp[row0[(size_t)g] + (int)(meta & 0xffffu)] : 0;
-            const size_t p0 = (size_t)step[(size_t)g * 4 + i / wave_rows];
-            for (int j = 0; j < len; ++j) {
-                const size_t st = p0 + j / lanes;
-                const int q = (i % wave_rows) * lanes + j % lanes;
-                col[st * 64 + q] = m->b4csr_col_id[k0 + j];
-                for (int e = 0; e < B; ++e)
-                    std::memcpy(&data[((st * B + e) * 64 + q) * 4], m->b4csr_data + ((size_t)e * N4 + k0 + j) * 4, 16);
+    int rc = 0;
+    DevBuf dcol = p->space((size_t)steps * 256, &rc);
+    if (rc) return rc;
+    DevBuf ddata = p->space((size_t)steps * 1024 * B, &rc);
+    if (rc) return rc;
+    // laid out and uploaded in pieces, whole groups each
+    const int piece_steps = std::max(1, (int)(kUploadPiece / (1024 * (size_t)B)));
+    std::unique_ptr<int[]> col;
+    std::unique_ptr<float[]> data;
+    size_t room = 0;
+    for (int a = 0, end = 0; a < ng; a = end) {
+        const int s0 = step[(size_t)a * 4];
+        for (end = a + 1; end < ng && step[(size_t)end * 4 + 4] - s0 <= piece_steps;) ++end;
+        const size_t ns = (size_t)(step[(size_t)end * 4] - s0);
+        if (ns > room) {  // a group may be larger than a piece
+            room = std::max(ns, (size_t)std::min<long long>(steps, piece_steps));
+            col.reset(new (std::nothrow) int[room * 64]);
+            data.reset(new (std::nothrow) float[room * 64 * B * 4]);
+            if (!col || !data) return CLSPMV_E_NOMEM;
+        }
+#pragma omp parallel for schedule(static, 4) num_threads(omp_threads()) if (end - a > 16)
+        for (int g = a; g < end; ++g) {
+            const size_t g0 = (size_t)(step[(size_t)g * 4] - s0), g1 = (size_t)(step[(size_t)g * 4 + 4] - s0);
+            std::memset(col.get() + g0 * 64, 0, (g1 - g0) * 256);  // padding: block column 0
+            std::memset(data.get() + g0 * 64 * B * 4, 0, (g1 - g0) * 1024 * B);
+            for (int i = 0; i < cap; ++i) {
+                const unsigned meta = lane[(size_t)g * cap + i];
+                const int len = (int)(meta >> 16);
+                if (!len) break;  // the group's last row with blocks is behind
+                const int k0 = rp[row0[(size_t)g] + (int)(meta & 0xffffu)];
+                size_t st = (size_t)(step[(size_t)g * 4 + i / wave_rows] - s0);
+                const int q0 = i % wave_rows * lanes;
+                for (int j = 0, t = 0; j < len; ++j) {
+                    col[st * 64 + q0 + t] = m->b4csr_col_id[k0 + j];
+                    for (int e = 0; e < B; ++e)
+                        std::memcpy(&data[((st * B + e) * 64 + q0 + t) * 4],
+                                    m->b4csr_data + ((size_t)e * N4 + k0 + j) * 4, 16);
+                    if (++t == lanes) t = 0, ++st;
+                }
             }
         }
+        rc = dcol.put(ctx, (size_t)s0 * 256, col.get(), ns * 256);
+        if (!rc) rc = ddata.put(ctx, (size_t)s0 * 1024 * B, data.get(), ns * 1024 * B);
+        if (rc) return rc;
     }
     DevBcsr d{};
-    int rc = 0;
     auto up = [&](const void* h, size_t bytes) -> const void* { return rc ? nullptr : p->add(ctx, h, bytes, &rc); };
     d.row_ptr = (const int*)up(row0.data(), (size_t)ng * 4);
     d.step = (const int*)up(step.data(), step.size() * 4);
     d.lane = (const unsigned*)up(lane.data(), (size_t)ng * cap * 4);
-    d.col = (const int*)up(col.get(), (size_t)steps * 256);
-    d.data = (const float*)up(data.get(), (size_t)steps * 1024 * B);
+    d.col = (const int*)dcol.ptr;
+    d.data = (const float*)ddata.ptr;
     if (rc) return rc;
     d.brows = brows;
     d.bh = bh;

@@ -24,6 +24,7 @@ struct DevBuf {
     size_t size = 0;
     int upload(clspmv_ctx_t ctx, const void* host, size_t bytes);
     int alloc(size_t bytes);
+    int put(clspmv_ctx_t ctx, size_t at, const void* host, size_t bytes);  // bytes of host to ptr + at, waits
     void release();
 };
 
