@@ -769,7 +769,8 @@ constexpr long long kCsrStagePays = 2;
 // in 16 (1.5 times) 48.9 and 43.8.  Several lanes per row round each row up to
 // 2 lanes entries, but their matrices are small and wait for one row's chain:
 // half as many bytes again are taken there (3000 rows of 1..64, 1.14 times:
-// 3.2 and 4.0 us; 30,000 with one of 64 in 16, 1.35 times: 3.8 and 3.5).
+// 3.2 and 4.0 us; 30,000 with one of 64 in 16, 1.35 times: 3.8 and 3.5), as
+// for a group with too few rows to sort into even waves (a matrix' last).
 constexpr double kCsrPadOne = 1.0, kCsrPadLanes = 1.5;
 
 // A row's l entries from its first lane's place on: two to a lane, lane by
@@ -866,7 +867,7 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
         d.xn = hi - d.x0 + 1;
         d.mode = d.xn <= kCsrWindow && d.xn <= kCsrStagePays * gn ? kCsrStaged : d.xn <= 65536 ? kCsrNear : kCsrWide;
         const bool wide = d.mode == kCsrWide;
-        stream[(size_t)g] = slots * (wide ? 8 : 6) > (8 * gn + 4 * gr) * (lanes > 1 ? kCsrPadLanes : kCsrPadOne);
+        stream[(size_t)g] = slots * (wide ? 8 : 6) > (8 * gn + 4 * gr) * (lanes > 1 || gr < cap ? kCsrPadLanes : kCsrPadOne);
     }
     // the rows of such groups become blocks; the others close ranks
     std::vector<std::pair<int, int>> stream_rows;
