@@ -87,7 +87,7 @@ __device__ __forceinline__ void csr_products(const int* __restrict__ col, const 
         if (lane + 64 * u < n) sh[lane + 64 * u] = v[u];
 }
 
-// One block of rows (csr_adaptive's and csr_slice's), by one wave:
+// One block of rows (csr_adaptive_kernel's and csr_blocks_kernel's), by one wave:
 //   {row, -(slot + 1)}  LONG, one chunk of a row: its sum to carry[slot]
 //   {row, row + 1}      VECTOR, one row
 //   {r0, r1}            STREAM, up to 64 rows of together at most
@@ -153,23 +153,19 @@ __device__ __forceinline__ void csr_block(int4 blk, const unsigned char* __restr
 }
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef int i32x2 __attribute__((ext_vector_type(2)));
 
 // kCsrPairs pairs of a wave from pair p on (those past the wave's last are
 // skipped, wave-uniform): two values and two columns per lane and pair.
-template <int MODE>
 struct CsrPairs {
-    typedef typename std::conditional<MODE == kCsrWide, i32x2, unsigned>::type C;
     f32x2 v[kCsrPairs];
-    C c[kCsrPairs];
-    __device__ __forceinline__ void load(const f32x2* __restrict__ val, const char* __restrict__ col, int p, int pairs,
-                                         int lane) {
-        const C* cp = reinterpret_cast<const C*>(col);
+    unsigned c[kCsrPairs];
+    __device__ __forceinline__ void load(const f32x2* __restrict__ val, const unsigned* __restrict__ col, int p,
+                                         int pairs, int lane) {
 #pragma unroll
         for (int u = 0; u < kCsrPairs; ++u)
             if (p + u < pairs) {
                 v[u] = __builtin_nontemporal_load(val + (size_t)(p + u) * 64 + lane);
-                c[u] = __builtin_nontemporal_load(cp + (size_t)(p + u) * 64 + lane);
+                c[u] = __builtin_nontemporal_load(col + (size_t)(p + u) * 64 + lane);
             }
     }
 };
@@ -179,9 +175,9 @@ struct CsrPairs {
 // row's length are padding (column 0 of the range, value 0) and multiply 0,
 // not x, so that an infinity or NaN of x they do not belong to stays out of
 // the sum.
-template <int L, int MODE>
-__device__ __forceinline__ float csr_group_sum(CsrPairs<MODE>& cur, const f32x2* __restrict__ val,
-                                               const char* __restrict__ col, int pairs, int len, int t, int lane,
+template <int L>
+__device__ __forceinline__ float csr_group_sum(CsrPairs& cur, const f32x2* __restrict__ val,
+                                               const unsigned* __restrict__ col, int pairs, int len, int t, int lane,
                                                const float* xg) {
     float acc = 0.f;
     int left = len - 2 * t;  // entries of the row from this lane's first on
@@ -191,13 +187,8 @@ __device__ __forceinline__ float csr_group_sum(CsrPairs<MODE>& cur, const f32x2*
 #pragma unroll
         for (int u = 0; u < kCsrPairs; ++u)
             if (p + u < pairs) {
-                if constexpr (MODE == kCsrWide) {
-                    xa[u] = xg[cur.c[u].x];
-                    xb[u] = xg[cur.c[u].y];
-                } else {
-                    xa[u] = xg[cur.c[u] & 0xffffu];
-                    xb[u] = xg[cur.c[u] >> 16];
-                }
+                xa[u] = xg[cur.c[u] & 0xffffu];
+                xb[u] = xg[cur.c[u] >> 16];
             }
 #pragma unroll
         for (int u = 0; u < kCsrPairs; ++u)
@@ -213,9 +204,8 @@ __device__ __forceinline__ float csr_group_sum(CsrPairs<MODE>& cur, const f32x2*
 // L lanes per row.  A workgroup of kCsrThreads threads owns one row group:
 // kCsrThreads / L rows of at most 64 entries, the longest first, so that the
 // 64 / L rows of a wave have nearly equal lengths; the wave's entries are
-// stored pair by pair, 64 lanes side by side (8 + 4 bytes per lane and pair
-// when the group's columns span at most 65536, else 8 + 8).  The x range of
-// the group is staged in LDS when it fits (kCsrWindow).
+// stored pair by pair, 64 lanes side by side (8 + 4 bytes per lane and pair).
+// The x range of the group is staged in LDS when it fits (kCsrWindow).
 // Bound by HBM on large matrices with columns near the diagonal: 1,000,003
 // rows of 9..27 entries within ~2000 columns (159 MB by CSR's count, 126 MB
 // stored) take 26.0 us, 6.1 TB/s of CSR bytes.  Waves that staged 512
@@ -234,7 +224,9 @@ __global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptiv
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     if ((int)blockIdx.x < nblock_wg) {
-        // few blocks: a CU each (blocks_per_wg of the waves take one)
+        // few blocks: spread over the CUs (blocks_per_wg of the waves take
+        // one).  Many: all waves, as a workgroup holds the groups' LDS (four
+        // of eight: 100,000 rows of 30 or 70 20.3 -> 24.8 us)
         const int b = blockIdx.x * blocks_per_wg + wave;
         if (wave < blocks_per_wg && b < m.nblocks)
             csr_block(m.blocks[b], m.counts, m.col, m.val, x, y, m.carry, xs + wave * kCsrStreamMaxNnz, lane);
@@ -250,13 +242,12 @@ __global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptiv
     const bool out = t == 0 && len > 0;
     const float yo = out ? *yp : 0.f;
     const f32x2* val = reinterpret_cast<const f32x2*>(m.gval) + (size_t)p0 * 64;
-    const char* col = reinterpret_cast<const char*>(m.gcol) +
-                      ((size_t)d.col256 + (size_t)(p0 - d.pair0) * (d.mode == kCsrWide ? 2 : 1)) * 256;
+    const unsigned* col = m.gcol + (size_t)p0 * 64;
+    CsrPairs first;
+    first.load(val, col, 0, pairs, lane);  // in flight while x is staged
+    const float* src = x + d.x0;
     float acc;
     if (d.mode == kCsrStaged) {
-        CsrPairs<kCsrStaged> first;
-        first.load(val, col, 0, pairs, lane);  // in flight while x is staged
-        const float* src = x + d.x0;
         for (int i = threadIdx.x * 4; i < d.xn; i += kCsrThreads * 4) {
             if (i + 4 <= d.xn) {
                 const f32x4a4 q = *reinterpret_cast<const f32x4a4*>(src + i);
@@ -268,28 +259,23 @@ __global__ __launch_bounds__(kCsrThreads) void csr_adaptive_kernel(DevCsrAdaptiv
             }
         }
         __syncthreads();
-        acc = csr_group_sum<L, kCsrStaged>(first, val, col, pairs, len, t, lane, xs);
-    } else if (d.mode == kCsrNear) {
-        CsrPairs<kCsrNear> first;
-        first.load(val, col, 0, pairs, lane);
-        acc = csr_group_sum<L, kCsrNear>(first, val, col, pairs, len, t, lane, x + d.x0);
+        acc = csr_group_sum<L>(first, val, col, pairs, len, t, lane, xs);
     } else {
-        CsrPairs<kCsrWide> first;
-        first.load(val, col, 0, pairs, lane);
-        acc = csr_group_sum<L, kCsrWide>(first, val, col, pairs, len, t, lane, x);
+        acc = csr_group_sum<L>(first, val, col, pairs, len, t, lane, src);
     }
     acc = group_sum<L>(acc);
     if (out) *yp = yo + acc;
 }
 
-// One column slice of the column-sliced CSR, in blocks of rows.  All x reads
-// of a launch fall in one slice of columns, small enough to stay in L2 while
-// the entry streams pass through with nontemporal loads.
-__global__ __launch_bounds__(256) void csr_slice_kernel(const unsigned char* __restrict__ counts,
-                                                        const int* __restrict__ col, const float* __restrict__ val,
-                                                        const int4* __restrict__ blocks, int nblocks,
-                                                        const float* __restrict__ x, float* __restrict__ y,
-                                                        double* __restrict__ carry) {
+// Blocks of rows by themselves: an adaptive layout without groups, or one
+// column slice of the column-sliced CSR, where all x reads of a launch fall in
+// one slice of columns, small enough to stay in L2 while the entry streams
+// pass through with nontemporal loads.
+__global__ __launch_bounds__(256) void csr_blocks_kernel(const unsigned char* __restrict__ counts,
+                                                         const int* __restrict__ col, const float* __restrict__ val,
+                                                         const int4* __restrict__ blocks, int nblocks,
+                                                         const float* __restrict__ x, float* __restrict__ y,
+                                                         double* __restrict__ carry) {
     __shared__ float lds[4][kCsrStreamMaxNnz];
     const int wid = threadIdx.x >> 6;
     const int b = blockIdx.x * 4 + wid;
@@ -344,7 +330,12 @@ static void csr_adaptive_launch(const DevCsrAdaptive& m, const float* x, float* 
 }
 
 int launch_csr_adaptive(const DevCsrAdaptive& m, const float* x, float* y, hipStream_t st) {
-    if (m.nblocks > 0 || m.ngroups > 0) {
+    if (m.ngroups == 0 && m.nblocks > 0) {
+        hipLaunchKernelGGL(dev::csr_blocks_kernel, dim3((m.nblocks + 3) / 4), dim3(256), 0, st, m.counts, m.col, m.val,
+                           m.blocks, m.nblocks, x, y, m.carry);
+        int e = (int)hipGetLastError();
+        if (e) return e;
+    } else if (m.ngroups > 0) {
         switch (m.lanes) {
             case 1: csr_adaptive_launch<1>(m, x, y, st); break;
             case 2: csr_adaptive_launch<2>(m, x, y, st); break;
@@ -367,7 +358,7 @@ int launch_csr_sliced(const DevCsrSliced& m, const float* x, float* y, hipStream
     for (int s = 0; s < m.nslices; ++s) {
         const int b0 = m.slice_block_begin[s], nb = m.slice_block_begin[s + 1] - b0;
         if (nb == 0) continue;
-        hipLaunchKernelGGL(dev::csr_slice_kernel, dim3((nb + 3) / 4), dim3(256), 0, st, m.counts + (size_t)s * m.rows,
+        hipLaunchKernelGGL(dev::csr_blocks_kernel, dim3((nb + 3) / 4), dim3(256), 0, st, m.counts + (size_t)s * m.rows,
                            m.col, m.val, m.blocks + b0, nb, x, y, m.carry);
         int e = (int)hipGetLastError();
         if (e) return e;

@@ -25,28 +25,27 @@ struct DevCsr {
 };
 // Adaptive CSR (k_csr.hip): rows of 1..kCsrStreamMaxRowLen entries in row
 // groups of one workgroup each, longer rows and the rows of groups that would
-// be mostly padding in blocks of one wave each.
+// be mostly padding or whose columns lie too far apart in blocks of one wave
+// each.
 constexpr int kCsrThreads = 512;
 constexpr int kCsrWaves = kCsrThreads / 64;
 constexpr int kCsrPairs = 4;          // entry pairs per lane in flight
-// How a group finds x: staged in LDS (16-bit columns into a range of at
-// most kCsrWindow), read from memory by 16-bit columns from x0, or by int32
-// columns.
-constexpr int kCsrStaged = 0, kCsrNear = 1, kCsrWide = 2;
+// How a group finds x by its 16-bit columns from x0: staged in LDS (a range of
+// at most kCsrWindow) or read from memory.
+constexpr int kCsrStaged = 0, kCsrNear = 1;
+constexpr int kCsrSpan = 65536;       // columns a group may span
 constexpr int kCsrWindow = 10240;     // floats: 40 KiB, four workgroups (32 waves) per CU
 struct CsrGroup {
     int row0;     // rows are stored as 16-bit offsets from it
-    int x0, xn;   // column range of the group (kCsrStaged, kCsrNear)
+    int x0, xn;   // column range of the group
     int mode;
-    int pair0;    // first pair of the group's first wave
-    int col256;   // its columns' offset in gcol, in units of 256 bytes
 };
 struct DevCsrAdaptive {
     const CsrGroup* groups;
     const int* pair;          // first pair of every wave (ngroups * kCsrWaves + 1)
     const unsigned* lane;     // per row: length << 16 | row - row0 (kCsrThreads / lanes per group)
     const float* gval;        // 64 lanes x 2 values per pair
-    const void* gcol;         // 64 lanes x 2 columns per pair, 16 or 32 bits each
+    const unsigned* gcol;     // 64 lanes x 2 columns of 16 bits per pair
     int ngroups, lanes;       // lanes per row: 1, 2, 4, 8 or 16
     int lds_floats;           // the widest staged x range, or the STREAM blocks' products
     // blocks {r0, r1 or -(slot + 1), n0, n1}, entries n0 .. n1 - 1 of col / val

@@ -764,25 +764,25 @@ constexpr long long kCsrStagePays = 2;
 // groups and blocks: lengths 1..16 (0.75 times CSR's bytes) 14.0 and 18.7 us,
 // one row of 64 in 16, the others of 2 (1.15 times) 17.8 and 15.3, power-law
 // lengths of exponent 1.8 (1.4 times) 18.5 and 15.4, one row of 64 in 512 rows
-// of 1 (4.5 times) 17.4 and 7.0.  With columns all over (int32 each) lengths
-// 1..16 (1.0 times) 62.5 and 59.4, 1..64 (1.09 times) 214 and 206, one of 64
-// in 16 (1.5 times) 48.9 and 43.8.  Several lanes per row round each row up to
+// of 1 (4.5 times) 17.4 and 7.0.  Several lanes per row round each row up to
 // 2 lanes entries, but their matrices are small and wait for one row's chain:
 // half as many bytes again are taken there (3000 rows of 1..64, 1.14 times:
 // 3.2 and 4.0 us; 30,000 with one of 64 in 16, 1.35 times: 3.8 and 3.5), as
 // for a group with too few rows to sort into even waves (a matrix' last).
+// Groups whose columns span more than 16 bits are blocks too: with int32
+// columns they waited for x like the blocks and took a little longer (1M rows
+// of 1..16 columns all over 62.5 and 59.4 us, 200,000 of 1..64 47.5 and 40.6).
 constexpr double kCsrPadOne = 1.0, kCsrPadLanes = 1.5;
 
 // A row's l entries from its first lane's place on: two to a lane, lane by
 // lane, then on to the wave's next pair.
-template <class Col>
-void csr_lay_row(const float* v, const int* c, int l, int lanes, int x0, float* val, Col* col) {
+void csr_lay_row(const float* v, const int* c, int l, int lanes, int x0, float* val, uint16_t* col) {
     for (int j = 0, t = 0; j < l; j += 2) {
         val[2 * t] = v[j];
-        col[2 * t] = (Col)(c[j] - x0);
+        col[2 * t] = (uint16_t)(c[j] - x0);
         if (j + 1 < l) {
             val[2 * t + 1] = v[j + 1];
-            col[2 * t + 1] = (Col)(c[j + 1] - x0);
+            col[2 * t + 1] = (uint16_t)(c[j + 1] - x0);
         }
         if (++t == lanes) {
             t = 0;
@@ -865,9 +865,9 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
         d.row0 = row0;
         d.x0 = lo & ~3;  // staged in 16-byte loads
         d.xn = hi - d.x0 + 1;
-        d.mode = d.xn <= kCsrWindow && d.xn <= kCsrStagePays * gn ? kCsrStaged : d.xn <= 65536 ? kCsrNear : kCsrWide;
-        const bool wide = d.mode == kCsrWide;
-        stream[(size_t)g] = slots * (wide ? 8 : 6) > (8 * gn + 4 * gr) * (lanes > 1 || gr < cap ? kCsrPadLanes : kCsrPadOne);
+        d.mode = d.xn <= kCsrWindow && d.xn <= kCsrStagePays * gn ? kCsrStaged : kCsrNear;
+        const double most = lanes > 1 || gr < cap ? kCsrPadLanes : kCsrPadOne;
+        stream[(size_t)g] = d.xn > kCsrSpan || 6 * slots > (8 * gn + 4 * gr) * most;
     }
     // the rows of such groups become blocks; the others close ranks
     std::vector<std::pair<int, int>> stream_rows;
@@ -888,61 +888,45 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
     groups.resize((size_t)ng);
     lane.resize((size_t)std::max(1, ng) * cap);
     pair.resize((size_t)ng * kCsrWaves + 1);
-    long long pairs = 0, col256 = 0;
+    long long pairs = 0;  // fits an int: the groups' bytes are bounded by their entries'
+    for (size_t i = 1; i < pair.size(); ++i) pair[i] = (int)(pairs += pair[i]);
     int lds_floats = stream_rows.empty() ? 0 : kCsrWaves * kCsrStreamMaxNnz;
-    for (int g = 0; g < ng; ++g) {
-        groups[(size_t)g].pair0 = (int)pairs;
-        groups[(size_t)g].col256 = (int)col256;
-        const long long p0 = pairs;
-        for (int w = 0; w < kCsrWaves; ++w) {
-            pairs += pair[(size_t)g * kCsrWaves + w + 1];
-            pair[(size_t)g * kCsrWaves + w + 1] = (int)pairs;
-        }
-        col256 += (pairs - p0) * (groups[(size_t)g].mode == kCsrWide ? 2 : 1);
-        if (groups[(size_t)g].mode == kCsrStaged) lds_floats = std::max(lds_floats, (groups[(size_t)g].xn + 3) & ~3);
-        if (col256 > INT32_MAX) return CLSPMV_E_TOO_LARGE;
-    }
+    for (const CsrGroup& d : groups)
+        if (d.mode == kCsrStaged) lds_floats = std::max(lds_floats, (d.xn + 3) & ~3);
     // the groups' entries, laid out and uploaded in pieces of kUploadPiece
     int rc = 0;
     DevBuf dval = p->space((size_t)pairs * 512, &rc);
     if (rc) return rc;
-    DevBuf dcol = p->space((size_t)col256 * 256, &rc);
+    DevBuf dcol = p->space((size_t)pairs * 256, &rc);
     if (rc) return rc;
     constexpr int piece_pairs = (int)(kUploadPiece / 512), group_pairs = kCsrWaves * kCsrStreamMaxRowLen / 2;
     const size_t room = (size_t)std::min<long long>(pairs, piece_pairs + group_pairs);
     std::unique_ptr<float[]> gval(new (std::nothrow) float[std::max<size_t>(1, room * 128)]);
-    std::unique_ptr<char[]> gcol(new (std::nothrow) char[std::max<size_t>(1, room * 512)]);
+    std::unique_ptr<uint16_t[]> gcol(new (std::nothrow) uint16_t[std::max<size_t>(1, room * 128)]);
     if (!gval || !gcol) return CLSPMV_E_NOMEM;
     for (int a = 0, b = 0; a < ng; a = b) {
         auto first_pair = [&](int g) { return pair[(size_t)g * kCsrWaves]; };
         for (b = a + 1; b < ng && first_pair(b) - first_pair(a) < piece_pairs;) ++b;
-        const CsrGroup& da = groups[(size_t)a];
-        const long long col_end = b < ng ? groups[(size_t)b].col256 : col256;
+        const int pa = first_pair(a);
 #pragma omp parallel for schedule(static, 4) num_threads(omp_threads()) if (b - a > 16)
         for (int g = a; g < b; ++g) {
             const CsrGroup& d = groups[(size_t)g];
-            const bool wide = d.mode == kCsrWide;
-            float* val = gval.get() + (size_t)(d.pair0 - da.pair0) * 128;
-            char* col = gcol.get() + (size_t)(d.col256 - da.col256) * 256;
-            const size_t np = (size_t)(first_pair(g + 1) - d.pair0);
-            std::memset(val, 0, np * 512);
-            std::memset(col, 0, np * (wide ? 512 : 256));  // padding: column 0 (wide) or x0
+            const size_t g0 = (size_t)(first_pair(g) - pa), g1 = (size_t)(first_pair(g + 1) - pa);
+            std::memset(gval.get() + g0 * 128, 0, (g1 - g0) * 512);
+            std::memset(gcol.get() + g0 * 128, 0, (g1 - g0) * 256);  // padding: column x0
             for (int i = 0; i < cap; ++i) {
                 const unsigned meta = lane[(size_t)g * cap + i];
                 const int l = (int)(meta >> 16);
                 if (!l) break;  // the group's last row is behind
                 const int k0 = rp[d.row0 + (int)(meta & 0xffffu)];
-                const size_t p0 = (size_t)(pair[(size_t)g * kCsrWaves + i / wave_rows] - d.pair0);
+                const size_t p0 = (size_t)(pair[(size_t)g * kCsrWaves + i / wave_rows] - pa);
                 const size_t q = (p0 * 64 + (size_t)(i % wave_rows) * lanes) * 2;
-                if (wide)
-                    csr_lay_row(cv + k0, ci + k0, l, lanes, 0, val + q, reinterpret_cast<int*>(col) + q);
-                else
-                    csr_lay_row(cv + k0, ci + k0, l, lanes, d.x0, val + q, reinterpret_cast<uint16_t*>(col) + q);
+                csr_lay_row(cv + k0, ci + k0, l, lanes, d.x0, gval.get() + q, gcol.get() + q);
             }
         }
-        rc = dval.put(ctx, (size_t)da.pair0 * 512, gval.get(), (size_t)(first_pair(b) - da.pair0) * 512);
-        if (!rc)
-            rc = dcol.put(ctx, (size_t)da.col256 * 256, gcol.get(), (size_t)(col_end - da.col256) * 256);
+        const size_t np = (size_t)(first_pair(b) - pa);
+        rc = dval.put(ctx, (size_t)pa * 512, gval.get(), np * 512);
+        if (!rc) rc = dcol.put(ctx, (size_t)pa * 256, gcol.get(), np * 256);
         if (rc) return rc;
     }
     // the blocks, over their rows' entries only
@@ -1022,7 +1006,7 @@ int build_csr_adaptive(clspmv_ctx_t ctx, clspmv_part_t p, const int* rp, const i
     d.pair = (const int*)up(pair.data(), pair.size() * 4);
     d.lane = (const unsigned*)up(lane.data(), lane.size() * 4);
     d.gval = (const float*)dval.ptr;
-    d.gcol = dcol.ptr;
+    d.gcol = (const unsigned*)dcol.ptr;
     d.col = (const int*)dlcol.ptr;
     d.val = (const float*)dlval.ptr;
     if (!counts.empty()) d.counts = (const unsigned char*)up(counts.data(), counts.size());
