@@ -9,7 +9,7 @@
 //    block's float4 column (guarded at the right matrix edge).
 //  * BCSR: the reference gives every block row a 128-thread workgroup with an
 //    LDS tree reduction (A/kernels/spmv_bcsr.cl:4-44).  Here block rows are
-//    regrouped at upload (bcsr_group_kernel: one to eight lanes per block
+//    regrouped at upload (bcsr_group_kernel: one to sixteen lanes per block
 //    row, 64 lanes' blocks side by side, rows of similar length in a wave);
 //    a part with a few block rows far longer than the rest keeps the arrays
 //    as they are, L lanes striding a block row (bcsr_kernel).
@@ -141,7 +141,7 @@ __global__ __launch_bounds__(256) void bcsr_kernel(const int* __restrict__ rp, c
 // EDGE: some block reaches past the last column (x guarded there).
 // Bound by HBM (250,000 block rows of nine 4 x 4 blocks 48 -> 25 us, 6.4
 // TB/s), smaller parts by the chain column -> x of a step (100,003 block
-// rows 22.2 -> 14.0), against 8 lanes striding each row's blocks as bcsr_kernel
+// rows 22.2 -> 12.8), against 8 lanes striding each row's blocks as bcsr_kernel
 // does: of nine blocks its second round used one lane, and one step's loads
 // were in flight.  Three steps at once measured 1-5 % ahead of four and five;
 // plain loads 15 % ahead of nontemporal ones.
@@ -447,15 +447,23 @@ static void launch_bcsr_groups(const DevBcsr& m, const float* x, float* y, hipSt
 #define CLSPMV_BCSR_GROUPS(L, E)                                                                                    \
     hipLaunchKernelGGL((dev::bcsr_group_kernel<BH, W4, L, E>), dim3(m.ngroups), dim3(256), 0, st, m.row_ptr, m.step, \
                        m.lane, m.col, d4, x, y, m.rows, m.cols)
-    switch (m.lanes + (m.edge ? 16 : 0)) {
-        case 1: CLSPMV_BCSR_GROUPS(1, false); break;
-        case 2: CLSPMV_BCSR_GROUPS(2, false); break;
-        case 4: CLSPMV_BCSR_GROUPS(4, false); break;
-        case 8: CLSPMV_BCSR_GROUPS(8, false); break;
-        case 17: CLSPMV_BCSR_GROUPS(1, true); break;
-        case 18: CLSPMV_BCSR_GROUPS(2, true); break;
-        case 20: CLSPMV_BCSR_GROUPS(4, true); break;
-        default: CLSPMV_BCSR_GROUPS(8, true); break;
+    switch (m.lanes * 2 + (m.edge ? 1 : 0)) {
+        case 2: CLSPMV_BCSR_GROUPS(1, false); break;
+        case 3: CLSPMV_BCSR_GROUPS(1, true); break;
+        case 4: CLSPMV_BCSR_GROUPS(2, false); break;
+        case 5: CLSPMV_BCSR_GROUPS(2, true); break;
+        case 8: CLSPMV_BCSR_GROUPS(4, false); break;
+        case 9: CLSPMV_BCSR_GROUPS(4, true); break;
+        case 16: CLSPMV_BCSR_GROUPS(8, false); break;
+        case 17: CLSPMV_BCSR_GROUPS(8, true); break;
+        default:  // 16 lanes: blocks of at least 8 float4 only
+            if constexpr (BH * W4 >= 8) {
+                if (m.edge)
+                    CLSPMV_BCSR_GROUPS(16, true);
+                else
+                    CLSPMV_BCSR_GROUPS(16, false);
+            }
+            break;
     }
 #undef CLSPMV_BCSR_GROUPS
 }

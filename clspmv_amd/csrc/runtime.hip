@@ -1841,10 +1841,14 @@ static bool bcsr_regroups(const int* rp, int brows) {
 }
 
 // Lanes per block row: doubled while the rows alone give fewer than
-// kBcsrFillWaves wavefronts and a row still feeds its lanes two blocks each
-// (2048, 4096 and 8192: 14.0, 15.2 and 15.2 us at 100,003 rows of nine
-// blocks, 9.6, 10.5 and 10.4 at 40,000 of sixteen).
-static constexpr long long kBcsrFillWaves = 2048;
+// kBcsrFillWaves wavefronts (1024, 2048, 4096 and 8192: 12.8, 14.1, 15.2 and
+// 15.2 us at 100,003 rows of nine 4 x 4 blocks) and a row still feeds its lanes
+// two blocks each, or one each of at least 8 x 4 or 4 x 8 values, of which a
+// lane has one or two in flight.  Rounding the mean up to the lanes must not
+// pad it too much (10,000 rows of nine 8 x 8: 6.2 us with 4 lanes, 9.0 plain),
+// but below a quarter of those wavefronts rounds count, not bytes, and where
+// that pads the plain layout is the faster one (3000 rows: 5.5 and 4.5).
+static constexpr long long kBcsrFillWaves = 1024;
 
 // Regroups the block rows into p; *padded (and p untouched) where that would
 // pad them too much.
@@ -1855,7 +1859,13 @@ static int build_bcsr_groups(clspmv_ctx_t ctx, clspmv_part_t p, const clspmv_b4c
     const int* rp = m->b4csr_row_ptr;
     const long long nb = rp[brows];
     int lanes = 1;
-    while (lanes < 8 && (long long)brows * lanes < 64 * kBcsrFillWaves && nb >= 4LL * lanes * brows) lanes *= 2;
+    const int most = B >= 8 ? 16 : 8, each = B >= 8 ? 1 : 2;
+    auto doubles = [&] {
+        const long long next = 2LL * lanes * brows, slots = (nb + next - 1) / std::max(1LL, next) * next;
+        return lanes < most && next < 128 * kBcsrFillWaves && nb >= each * next &&
+               (next < 32 * kBcsrFillWaves || slots <= kBcsrPad * nb);
+    };
+    while (doubles()) lanes *= 2;
     const int cap = 256 / lanes, wave_rows = 64 / lanes;
     const int ng = (brows + cap - 1) / cap;
     std::vector<int> row0((size_t)std::max(1, ng)), step((size_t)ng * 4 + 1, 0);

@@ -1,5 +1,5 @@
 """The regrouped BCSR kernel (k_block.hip: bcsr_group_kernel) at its edges:
-every block shape, one to eight lanes per block row, ragged and empty block
+every block shape, one to sixteen lanes per block row, ragged and empty block
 rows, a width that no block column divides, one group and one row more, and
 the parts that keep the plain kernel (a block row far longer than the rest, or
 skewed rows that regrouping would pad); padding next to an infinite x entry.  Tolerance: the FP32 bar of
@@ -54,6 +54,14 @@ def test_block_shapes(ctx, bh, bw, width):
 def test_lanes_per_block_row(ctx, rows, lo, hi, lanes):
     lens = np.random.default_rng(rows).integers(lo, hi + 1, rows)
     _check(ctx, _coo(lens, 1, 4, 1000, rows), 4, 1, f"_G{lanes}")
+
+
+@pytest.mark.parametrize("width", [804, 803])
+@pytest.mark.parametrize("bh,bw", [(8, 8), (8, 4), (4, 8)])
+def test_sixteen_lanes_per_block_row(ctx, bh, bw, width):
+    # blocks of eight float4 and more only: a block row feeds its lanes one each
+    lens = np.random.default_rng(bh * 10 + bw).integers(16, 34, 130)
+    _check(ctx, _coo(lens, bh, bw, width, bh + bw), bw, bh, "_G16")
 
 
 def test_one_long_block_row_keeps_the_plain_kernel(ctx):
