@@ -3,8 +3,9 @@
 // The reference splits the entries into per-workgroup ranges, runs an LDS
 // segmented scan with a barrier per step and folds the per-group carries in a
 // second one-workgroup kernel (A/kernels/spmv_coo.cl:4-200).  Here one
-// wavefront owns a 512-entry chunk and each lane owns 8 consecutive entries,
-// loaded as two dwordx4 per array (a wave's loads are contiguous):
+// wavefront owns a 512-entry chunk and each lane four consecutive entries of
+// each half of it, one dwordx4 per array and half (a wave's load is 1 KiB side
+// by side):
 //   1. each lane sums its entries since its last row break, and a segmented
 //      scan in DPP moves carries these tails into the next lanes;
 //   2. every break ends a segment: its sum and row go to the wave's LDS at

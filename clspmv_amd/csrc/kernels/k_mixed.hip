@@ -228,7 +228,7 @@ __global__ __launch_bounds__(256) void dia_mixed_kernel(const int* __restrict__ 
         for (int d = 0; d < ndiag; d += U) {
             unsigned w[U][W];
             float xv[U][R];
-    #pragma unroll
+#pragma unroll
             for (int u = 0; u < U; ++u)
                 if (d + u < ndiag) {
                     word(d + u, w[u]);
@@ -236,16 +236,16 @@ __global__ __launch_bounds__(256) void dia_mixed_kernel(const int* __restrict__ 
                     if (interior) {
                         load_x_run<R>(x, c, xv[u]);
                     } else {
-    #pragma unroll
+#pragma unroll
                         for (int j = 0; j < R; ++j) xv[u][j] = xload_m(x, c + j, cols);
                     }
                 }
-    #pragma unroll
+#pragma unroll
             for (int u = 0; u < U; ++u)
                 if (d + u < ndiag) {
                     float v[R];
                     dia_decode<CODEC, R, W>(w[u], slice_scale(d + u), v);
-    #pragma unroll
+#pragma unroll
                     for (int j = 0; j < R; ++j) a[j] = fmaf(v[j], xv[u][j], a[j]);
                 }
         }
